@@ -8,18 +8,13 @@
 // Rows with no live key have P = 0 and get no gradient.
 //
 // Tiles are 64 x 64 (query block x key block), from the block index built at
-// BQ = A = 64 and its transpose (pa_index_transpose).  Two passes, no atomics:
-//  * dK / dV, per (key block, head): S = Q K^T and dP = dO V^T come out with the keys
-//    along the lanes, and dV^T += dO^T P, dK^T += Q^T dS use transposed LDS reads of dO
-//    and Q.  D = 64: bwd_dkdv_kernel, 2 waves of 32 keys, tiles staged through registers.
-//    D = 128: bwd_dkdv_pair_kernel, 4 waves, a pair per 32 keys with the two products
-//    split between the pair's waves, tiles by LDS DMA.
-//  * dQ, per (query block, head), the same with the roles of queries and keys exchanged
-//    (the forward's layout): S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T.  D = 64:
-//    bwd_dq_kernel; D = 128: bwd_dq_stream_kernel (tiles by LDS DMA).
-// Partial tiles are masked from element bitmaps when given (D = 128), else by evaluating
-// the mask in original coordinates (perm_q / perm_kv map index-space rows to them, as in
-// the forward).
+// BQ = A = 64 and its transpose (pa_index_transpose).  Two passes, no atomics: dK / dV per
+// (key block, head), dQ per (query block, head), each a work-group that walks its list with
+// the next tile moving into LDS by DMA while the current one is consumed.  A wave owns one
+// 32 x 32 quadrant of every tile from the scores to the accumulators, so nothing passes
+// between waves inside a tile.
+// Partial tiles are masked from element bitmaps when given, else by evaluating the mask in
+// original coordinates (perm_q / perm_kv map index-space rows to them, as in the forward).
 #include <math.h>
 
 #include <type_traits>
@@ -60,7 +55,7 @@ struct BwdK {
   const int32_t* q_bits_off;   // [nb, tpitch], same offsets in the transposed lists
   const uint32_t* q_bits;      // the same bitmaps transposed (64 columns x 2 words)
   int32_t accumulate;          // add into dq / dk / dv
-  // > 0 (D = 128 only): the tensors (and lse, dvec) are in ORIGINAL order and index-space
+  // > 0: the tensors (and lse, dvec) are in ORIGINAL order and index-space
   // row r lives at row (r mod 2^qlog2) s + r div 2^qlog2 (the residue-s permutation in
   // closed form); a 64-row tile is then 64 rows s apart
   int32_t residue_s, residue_qlog2;
@@ -71,13 +66,6 @@ struct BwdK {
 // Memory row of index-space row r.
 __device__ __forceinline__ int64_t mem_row(const BwdK& a, int r) {
   return a.residue_s ? (int64_t)(r & ((1 << a.residue_qlog2) - 1)) * a.residue_s + (r >> a.residue_qlog2) : r;
-}
-
-// 4 gradient elements stored (or added to the stored ones) in the tensor's type.
-template <typename T>
-__device__ __forceinline__ void store_grad4(char* p, f32x4 x, bool acc) {
-  if (acc) x += load4_any(p, __is_same(T, __bf16) ? PA_BF16 : PA_F16);
-  Mma<T>::store4(p, x);
 }
 
 // rowsum(dO * O) in fp32: a row per D / 8 lanes, 16 bytes of each tensor per lane (the
@@ -106,620 +94,494 @@ __global__ __launch_bounds__(256) void bwd_pre_kernel(const BwdK a, int64_t rows
   }
 }
 
-// LDS pitches of a staged 64-row tile: the K-style pitch (+16 B) serves the 16-byte row
-// reads, the V-style pitch (+64 B) the transposed reads; a tile read both ways is
-// staged twice.
-template <typename T, int D>
-constexpr int npitch() { return D * (int)sizeof(T) + 16; }
-template <typename T, int D>
-constexpr int tpitch() { return D * (int)sizeof(T) + 64; }
-
-// Stage rows r0 .. r0 + 63 of a [BH, N, D] tensor into LDS at the row-read pitch and,
-// with TR, also at the transposed-read pitch.  128 threads; a fixed unit count per
-// thread, so every load is issued before any store.
-template <typename T, int D, bool TR>
-__device__ __forceinline__ void stage_tile(const char* base, int64_t sn, int r0, char* dst_n, char* dst_t, int tid) {
-  constexpr int UPR = D * (int)sizeof(T) / 16;
-  constexpr int PER = kBT * UPR / 128;
-  uint4 x[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int u = tid + 128 * i, r = u / UPR, c = u % UPR;
-    x[i] = *reinterpret_cast<const uint4*>(base + ((int64_t)(r0 + r) * sn) * (int64_t)sizeof(T) + 16 * c);
-  }
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int u = tid + 128 * i, r = u / UPR, c = u % UPR;
-    *reinterpret_cast<uint4*>(dst_n + r * npitch<T, D>() + 16 * c) = x[i];
-    if constexpr (TR) *reinterpret_cast<uint4*>(dst_t + r * tpitch<T, D>() + 16 * c) = x[i];
-  }
-}
-
-// Fragments of 16-byte row reads: lane (m, G) holds row m, bytes (16 kc + 8 G) * esz.
-template <typename T, int D>
-__device__ __forceinline__ void row_frags(const char* row, typename Mma<T>::frag* f) {
-#pragma unroll
-  for (int kc = 0; kc < D / 16; ++kc) f[kc] = __builtin_bit_cast(typename Mma<T>::frag, *reinterpret_cast<const uint4*>(row + kc * 32));
-}
-
-// A operand X^T[d][r] of a transposed product for rows 16 c + 4 G + 0..3 and
-// 16 c + 8 + 4 G + 0..3 of a tile staged at the V-style pitch (the rows whose values
-// this lane holds in elements 8 c .. 8 c + 7 of an accumulator): block db of D.
-template <typename T, int D>
-__device__ __forceinline__ typename Mma<T>::frag tr_frag(const char* tile_t, int lane, int G, int rbase, int db) {
-  constexpr int TP = tpitch<T, D>();
-  const int j16 = lane & 15;
-  const char* p = tile_t + (rbase + 4 * G + (j16 >> 2)) * TP + (((lane >> 4) & 1) * 16 + 4 * (j16 & 3)) * 2 + db * 64;
-  const s16x4 x1 = lds_read_tr(p);
-  const s16x4 x2 = lds_read_tr(p + 8 * TP);
-  const uint4 vx = {__builtin_bit_cast(uint2, x1).x, __builtin_bit_cast(uint2, x1).y, __builtin_bit_cast(uint2, x2).x,
-                    __builtin_bit_cast(uint2, x2).y};
-  return __builtin_bit_cast(typename Mma<T>::frag, vx);
-}
-
 __device__ __forceinline__ int32_t orig_of(const int32_t* perm, int32_t r) { return perm ? perm[r] : r; }
 
-// ---------------------------------------------------------------------------------
-template <typename T, int D>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1))) void bwd_dkdv_kernel(const BwdK a) {
-  using Frag = typename Mma<T>::frag;
-  constexpr int ESZ = sizeof(T);
-  constexpr int NKC = D / 16;
-  constexpr int NDB = D / 32;
-  constexpr int NP = npitch<T, D>();
-  constexpr int TP = tpitch<T, D>();
-  __shared__ __attribute__((aligned(16))) char q_n[kBT * NP];
-  __shared__ __attribute__((aligned(16))) char q_t[kBT * TP];
-  __shared__ __attribute__((aligned(16))) char do_n[kBT * NP];
-  __shared__ __attribute__((aligned(16))) char do_t[kBT * TP];
-  __shared__ float lse_s[kBT], dvec_s[kBT];
-  __shared__ int32_t qo_s[kBT];
-  __shared__ pa_term terms_s[PA_MAX_TERMS];
-#pragma unroll
-  for (int i = 0; i < PA_MAX_TERMS; ++i)  // (constant indices into the argument block)
-    if (threadIdx.x == i) terms_s[i] = a.pred.terms[i];
-
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, G = lane >> 5, m = lane & 31;
-  const int kb = blockIdx.x;
-  const int64_t bh = blockIdx.y;
-  const int key = kb * kBT + w * 32 + m;  // this lane's key (index space)
-  const int key_o = orig_of(a.pred.perm_kv, key);
-  const char* hq = a.q + bh * a.sb * ESZ;
-  const char* hdo = a.dout + bh * a.sb * ESZ;
-
-  Frag kf[NKC], vf[NKC];
-  row_frags<T, D>(a.k + (bh * a.sb + (int64_t)key * a.sn) * ESZ + 16 * G, kf);
-  row_frags<T, D>(a.v + (bh * a.sb + (int64_t)key * a.sn) * ESZ + 16 * G, vf);
-  f32x16 dkt[NDB], dvt[NDB];
-#pragma unroll
-  for (int i = 0; i < NDB; ++i) dkt[i] = dvt[i] = f32x16{0};
-
-  const int nl = a.q_num[kb];
-  for (int t = 0; t < nl; ++t) {
-    const int qb = a.q_idx[(int64_t)kb * a.tpitch + t];
-    const bool partial = a.q_partial[(int64_t)kb * a.tpitch + t] != 0;
-    __syncthreads();  // the previous block's tiles are consumed
-    stage_tile<T, D, true>(hq, a.sn, qb * kBT, q_n, q_t, tid);
-    stage_tile<T, D, true>(hdo, a.sn, qb * kBT, do_n, do_t, tid);
-    if (tid < kBT) {
-      const float l = a.lse[bh * a.lse_sb + qb * kBT + tid];
-      lse_s[tid] = l * 1.4426950408889634f;
-      dvec_s[tid] = a.dvec[bh * a.lse_sb + qb * kBT + tid];
-      qo_s[tid] = orig_of(a.pred.perm_q, qb * kBT + tid);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int lb = 0; lb < 2; ++lb) {
-      // S = Q K^T and dP = dO V^T for query rows 32 lb .. +31: element i of the lane is
-      // query row 32 lb + 8 (i / 4) + 4 G + i % 4, key `key`
-      f32x16 s = f32x16{0}, dp = f32x16{0};
-      const char* qrow = q_n + (32 * lb + m) * NP + 16 * G;
-      const char* drow = do_n + (32 * lb + m) * NP + 16 * G;
-#pragma unroll
-      for (int kc = 0; kc < NKC; ++kc) {
-        s = Mma<T>::mma(__builtin_bit_cast(Frag, *reinterpret_cast<const uint4*>(qrow + kc * 32)), kf[kc], s);
-        dp = Mma<T>::mma(__builtin_bit_cast(Frag, *reinterpret_cast<const uint4*>(drow + kc * 32)), vf[kc], dp);
-      }
-      // live bit i of the lane's elements: all set on a full tile, one rolled copy of the
-      // predicate (terms from LDS) on a partial one
-      uint32_t live = 0xffffu;
-      if (partial) {
-        live = 0u;
-#pragma unroll 1
-        for (int i = 0; i < 16; ++i) {
-          const int qr = 32 * lb + 8 * (i >> 2) + 4 * G + (i & 3);
-          if (pred_live_rolled(terms_s, a.pred.n_include, a.pred.n_exclude, qo_s[qr], key_o, a.pred.dense_bits,
-                               a.pred.dense_words))
-            live |= 1u << i;
-        }
-      }
-      float p[16], ds[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int qr = 32 * lb + 8 * (i >> 2) + 4 * G + (i & 3);
-        const float l2 = lse_s[qr];
-        p[i] = (((live >> i) & 1u) && l2 != -INFINITY) ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.c, -l2)) : 0.f;
-        ds[i] = p[i] * (dp[i] - dvec_s[qr]);
-      }
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        f32x8 pv, sv;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          pv[e] = p[8 * c + e];
-          sv[e] = ds[8 * c + e];
-        }
-        const Frag pf = Mma<T>::cvt(pv), sf = Mma<T>::cvt(sv);
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          dvt[db] = Mma<T>::mma(tr_frag<T, D>(do_t, lane, G, 32 * lb + 16 * c, db), pf, dvt[db]);
-          dkt[db] = Mma<T>::mma(tr_frag<T, D>(q_t, lane, G, 32 * lb + 16 * c, db), sf, dkt[db]);
-        }
-      }
-    }
+// ---- staged tiles ------------------------------------------------------------------
+// A tile of 64 rows of two tensors is brought into LDS by LDS DMA (no staging registers,
+// no LDS stores), two stages deep: the next listed tile moves while the current one is
+// consumed, behind one wait and one barrier per tile.  A DMA instruction writes 64
+// consecutive 16-byte units, so the rows are stored unpadded and one XOR swizzle of the
+// 16-byte units serves both ways a tile is read (unit u of row r sits at u ^ swz(r)):
+//  * D = 128 (256-byte rows): 4 (r % 4) + (r / 4) % 4.  The 16 rows of a 16-byte row read
+//    land on 16 different units of the 256-byte bank window, and the 4 rows of a transposed
+//    read on 4 different 64-byte groups;
+//  * D = 64 (128-byte rows, two to a bank window): with x = (r / 2) % 8, 4 (x % 2) + x / 2.
+//    The 8 row pairs of a row read land on 8 different units, and the two rows of one
+//    parity that a transposed read touches (x differing in its lowest bit) on different
+//    halves of the row.
+// LDS of both kernels: two stages of two tiles, then per stage 1 KB of row vectors (at 0 and
+// 256: two vectors of 64 floats; at 512: the partial tile's bitmap, or without bitmaps the
+// original numbers of the tile's rows, and in stage 0 at 768 the mask's terms).
+template <int D>
+struct Tile {
+  static constexpr int ROW = 2 * D;             // bytes of a row
+  static constexpr int UPR = D / 8;             // 16-byte units of a row
+  static constexpr int RPI = 64 / UPR;          // rows a DMA instruction moves
+  static constexpr int NI = 16 / RPI;           // instructions per tensor and wave (16 rows)
+  static constexpr int TB = kBT * ROW;          // bytes of a staged tile
+  static constexpr int STAGE = 2 * TB;
+  static constexpr int VEC = 1024;
+  static constexpr int VEC_OFF = 2 * STAGE;
+  static constexpr int TERMS_OFF = VEC_OFF + 768;
+  static constexpr int END = VEC_OFF + 2 * VEC;
+  static_assert(PA_MAX_TERMS * sizeof(pa_term) <= 256, "the terms fit beside the row numbers");
+  __device__ static int swz(int r) {
+    return D == 128 ? 4 * (r & 3) + ((r >> 2) & 3) : 4 * ((r >> 1) & 1) + ((r >> 2) & 3);
   }
-  // dK^T / dV^T blocks [32 d x 32 keys]: lane (key m, G) holds d = 32 db + 8 i4 + 4 G + 0..3
-  char* dkrow = a.dk + (bh * a.sb + (int64_t)key * a.sn) * ESZ;
-  char* dvrow = a.dv + (bh * a.sb + (int64_t)key * a.sn) * ESZ;
-#pragma unroll
-  for (int db = 0; db < NDB; ++db) {
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const int d0 = 32 * db + 8 * i4 + 4 * G;
-      f32x4 xk = {dkt[db][4 * i4], dkt[db][4 * i4 + 1], dkt[db][4 * i4 + 2], dkt[db][4 * i4 + 3]};
-      const f32x4 xv = {dvt[db][4 * i4], dvt[db][4 * i4 + 1], dvt[db][4 * i4 + 2], dvt[db][4 * i4 + 3]};
-      xk *= a.scale;
-      store_grad4<T>(dkrow + d0 * ESZ, xk, a.accumulate);
-      store_grad4<T>(dvrow + d0 * ESZ, xv, a.accumulate);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------
-template <typename T, int D>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void bwd_dq_kernel(const BwdK a) {
-  using Frag = typename Mma<T>::frag;
-  constexpr int ESZ = sizeof(T);
-  constexpr int NKC = D / 16;
-  constexpr int NDB = D / 32;
-  constexpr int NP = npitch<T, D>();
-  constexpr int TP = tpitch<T, D>();
-  __shared__ __attribute__((aligned(16))) char k_n[kBT * NP];
-  __shared__ __attribute__((aligned(16))) char k_t[kBT * TP];
-  __shared__ __attribute__((aligned(16))) char v_n[kBT * NP];
-  __shared__ int32_t ko_s[kBT];
-  __shared__ pa_term terms_s[PA_MAX_TERMS];
-#pragma unroll
-  for (int i = 0; i < PA_MAX_TERMS; ++i)
-    if (threadIdx.x == i) terms_s[i] = a.pred.terms[i];
-
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, G = lane >> 5, m = lane & 31;
-  const int qb = blockIdx.x;
-  const int64_t bh = blockIdx.y;
-  const int row = qb * kBT + w * 32 + m;  // this lane's query row (index space)
-  const int q_o = orig_of(a.pred.perm_q, row);
-  const char* hk = a.k + bh * a.sb * ESZ;
-  const char* hv = a.v + bh * a.sb * ESZ;
-
-  Frag qf[NKC], df[NKC];
-  row_frags<T, D>(a.q + (bh * a.sb + (int64_t)row * a.sn) * ESZ + 16 * G, qf);
-  row_frags<T, D>(a.dout + (bh * a.sb + (int64_t)row * a.sn) * ESZ + 16 * G, df);
-  const float l2 = a.lse[bh * a.lse_sb + row] * 1.4426950408889634f;
-  const float dr = a.dvec[bh * a.lse_sb + row];
-  f32x16 dqt[NDB];
-#pragma unroll
-  for (int i = 0; i < NDB; ++i) dqt[i] = f32x16{0};
-
-  const int nl = a.kv_num[qb];
-  for (int t = 0; t < nl; ++t) {
-    const int kb = a.kv_idx[(int64_t)qb * a.pitch + t];
-    const bool partial = a.kv_partial[(int64_t)qb * a.pitch + t] != 0;
-    __syncthreads();
-    stage_tile<T, D, true>(hk, a.sn, kb * kBT, k_n, k_t, tid);
-    stage_tile<T, D, false>(hv, a.sn, kb * kBT, v_n, nullptr, tid);
-    if (tid < kBT) ko_s[tid] = orig_of(a.pred.perm_kv, kb * kBT + tid);
-    __syncthreads();
-#pragma unroll
-    for (int lb = 0; lb < 2; ++lb) {
-      // S^T = K Q^T and dP^T = V dO^T for keys 32 lb .. +31: element i is key
-      // 32 lb + 8 (i / 4) + 4 G + i % 4, query `row`
-      f32x16 s = f32x16{0}, dp = f32x16{0};
-      const char* krow = k_n + (32 * lb + m) * NP + 16 * G;
-      const char* vrow = v_n + (32 * lb + m) * NP + 16 * G;
-#pragma unroll
-      for (int kc = 0; kc < NKC; ++kc) {
-        s = Mma<T>::mma(__builtin_bit_cast(Frag, *reinterpret_cast<const uint4*>(krow + kc * 32)), qf[kc], s);
-        dp = Mma<T>::mma(__builtin_bit_cast(Frag, *reinterpret_cast<const uint4*>(vrow + kc * 32)), df[kc], dp);
-      }
-      uint32_t live = 0xffffu;
-      if (partial) {
-        live = 0u;
-#pragma unroll 1
-        for (int i = 0; i < 16; ++i) {
-          const int kr = 32 * lb + 8 * (i >> 2) + 4 * G + (i & 3);
-          if (pred_live_rolled(terms_s, a.pred.n_include, a.pred.n_exclude, q_o, ko_s[kr], a.pred.dense_bits,
-                               a.pred.dense_words))
-            live |= 1u << i;
-        }
-      }
-      float ds[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const float p =
-            (((live >> i) & 1u) && l2 != -INFINITY) ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.c, -l2)) : 0.f;
-        ds[i] = p * (dp[i] - dr);
-      }
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        f32x8 sv;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sv[e] = ds[8 * c + e];
-        const Frag sf = Mma<T>::cvt(sv);
-#pragma unroll
-        for (int db = 0; db < NDB; ++db)
-          dqt[db] = Mma<T>::mma(tr_frag<T, D>(k_t, lane, G, 32 * lb + 16 * c, db), sf, dqt[db]);
-      }
-    }
-  }
-  char* dqrow = a.dq + (bh * a.sb + (int64_t)row * a.sn) * ESZ;
-#pragma unroll
-  for (int db = 0; db < NDB; ++db) {
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const int d0 = 32 * db + 8 * i4 + 4 * G;
-      f32x4 x = {dqt[db][4 * i4], dqt[db][4 * i4 + 1], dqt[db][4 * i4 + 2], dqt[db][4 * i4 + 3]};
-      x *= a.scale;
-      store_grad4<T>(dqrow + d0 * ESZ, x, a.accumulate);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------
-// D = 128 (f16 / bf16): the same two products per tile, with the staged tiles brought
-// into LDS by LDS DMA (no staging registers, no LDS stores), two stages deep: the next
-// listed tile moves while the current one is consumed, behind one wait and one barrier
-// per tile.  A DMA instruction writes 64 consecutive 16-byte units, so the rows are
-// stored unpadded (256 B) and one XOR swizzle of the 16-byte units serves both ways a
-// tile is read: unit u of row r sits at u ^ bswz(r), bswz(r) = 4 (r % 4) + (r / 4) % 4.
-// The 16 rows of a 16-byte row read land on 16 different units of the 256-byte bank
-// window, and the 4 rows of a transposed read on 4 different 64-byte groups.
-// LDS: two stages of two tiles, then per stage 2 KB of row vectors (lse, rowsum(dO O),
-// original row numbers; the partial tile's bitmap at +1 KB), then the mask terms.
-constexpr int kTB = kBT * 256;
-constexpr int kStage = 2 * kTB;
-constexpr int kVecOff = 2 * kStage;
-constexpr int kVec = 2048;
-constexpr int kBitsAt = 1024;
-constexpr int kTermsOff = kVecOff + 2 * kVec;
-constexpr int kBwdSmem = kTermsOff + PA_MAX_TERMS * (int)sizeof(pa_term);
+};
 
 typedef const __attribute__((address_space(3))) f32x4 lds_f4;
+typedef __attribute__((address_space(3))) f32x4 lds_f4w;
+typedef __attribute__((address_space(3))) u32x4 lds_u4w;
 typedef const __attribute__((address_space(3))) int32_t lds_i32;
-typedef const __attribute__((address_space(3))) u32x2 lds_u2;
+typedef __attribute__((address_space(3))) float lds_fw;
 typedef const __attribute__((address_space(4))) int32_t cint;
 typedef const __attribute__((address_space(4))) int8_t cbyte;
 
-__device__ __forceinline__ int bswz(int r) { return 4 * (r & 3) + ((r >> 2) & 3); }
-
-// Live bits of a score block's 16 elements (element i = row or column 8 (i / 4) + 4 G +
-// i % 4 of the 32 the bitmap word covers).
-__device__ __forceinline__ uint32_t live16(uint32_t word, int G) {
-  const uint32_t x = word >> (4 * G);
-  return (x & 0xfu) | ((x >> 4) & 0xf0u) | ((x >> 8) & 0xf00u) | ((x >> 12) & 0xf000u);
-}
-
-// Per-lane LDS geometry of a staged tile (offsets of stage, tile, block and chunk are
-// immediates on top of these).
+// Per-lane LDS geometry of the reads of 32 staged rows (offsets of stage, tile and chunk are
+// immediates on top of these).  With 256-byte rows, units 8 apart and blocks 2 apart differ
+// in address bit 7 alone, so the upper half of the addresses is the lower half with that
+// bit flipped: one VALU operation at the read instead of eight registers held through
+// the loop.
+template <int D>
 struct TileReads {
-  lds_cptr row[8];     // 16-byte row reads: row m, unit 2 kc + G
-  lds_cptr tr[4][2];   // transposed reads of block db: rows 4 G + j16 / 4 (+8)
+  static constexpr int NR = D == 128 ? 4 : D / 16, NT = 2;
+  lds_cptr row_[NR];     // 16-byte row reads: row m, unit 2 kc + G
+  lds_cptr tr_[NT][2];   // transposed reads of block db: rows 4 G + j16 / 4 (+8)
+  // (volatile, or the flips would be hoisted out of the loop into registers again)
+  __device__ __forceinline__ static lds_cptr flip(lds_cptr p) {
+    uint32_t x;
+    asm volatile("v_xor_b32 %0, 0x80, %1" : "=v"(x) : "v"((uint32_t)(uintptr_t)p));
+    return (lds_cptr)(uintptr_t)x;
+  }
+  __device__ __forceinline__ lds_cptr row(int kc) const { return kc < NR ? row_[kc] : flip(row_[kc - NR]); }
+  __device__ __forceinline__ lds_cptr tr(int db, int s) const { return db < NT ? tr_[db][s] : flip(tr_[db - NT][s]); }
 };
 
-__device__ __forceinline__ TileReads tile_reads(lds_cptr lds, int lane) {
-  TileReads t;
+template <int D>
+__device__ __forceinline__ TileReads<D> tile_reads(lds_cptr lds, int lane) {
+  TileReads<D> t;
   const int m = lane & 31, G = lane >> 5, j16 = lane & 15, h16 = (lane >> 4) & 1;
 #pragma unroll
-  for (int kc = 0; kc < 8; ++kc) {
-    t.row[kc] = lds + m * 256 + 16 * ((2 * kc + G) ^ bswz(m));
+  for (int kc = 0; kc < TileReads<D>::NR; ++kc) {
+    t.row_[kc] = lds + m * Tile<D>::ROW + 16 * ((2 * kc + G) ^ Tile<D>::swz(m));
     // (opaque, so each address stays whole in one register)
-    asm volatile("" : "+v"(t.row[kc]));
+    asm volatile("" : "+v"(t.row_[kc]));
   }
 #pragma unroll
-  for (int db = 0; db < 4; ++db)
+  for (int db = 0; db < TileReads<D>::NT; ++db)
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       const int R = 4 * G + (j16 >> 2) + 8 * s;
       const int u = 4 * db + 2 * h16 + ((j16 & 3) >> 1);
-      t.tr[db][s] = lds + R * 256 + 16 * (u ^ bswz(R)) + 8 * (j16 & 1);
-      asm volatile("" : "+v"(t.tr[db][s]));
+      t.tr_[db][s] = lds + R * Tile<D>::ROW + 16 * (u ^ Tile<D>::swz(R)) + 8 * (j16 & 1);
+      asm volatile("" : "+v"(t.tr_[db][s]));
     }
   return t;
 }
 
-// A operand X^T of rows r0 .. r0 + 15 (r0 a multiple of 16) of a staged tile at byte
-// offset `off` (stage + tile + r0 * 256): the transposed product's fragment for block db.
-template <typename T>
-__device__ __forceinline__ typename Mma<T>::frag tr_frag_sw(const TileReads& t, int db, int off) {
-  const s16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t.tr[db][0] + off));
-  const s16x4 x2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t.tr[db][1] + off));
+// A operand X^T of 16 rows of a staged tile at byte offset `off` (stage + tile + first row):
+// the transposed product's fragment for block db of D.
+template <typename T, int D>
+__device__ __forceinline__ typename Mma<T>::frag tr_frag(const TileReads<D>& t, int db, int off) {
+  const s16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t.tr(db, 0) + off));
+  const s16x4 x2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t.tr(db, 1) + off));
   const uint4 vx = {__builtin_bit_cast(uint2, x1).x, __builtin_bit_cast(uint2, x1).y, __builtin_bit_cast(uint2, x2).x,
                     __builtin_bit_cast(uint2, x2).y};
   return __builtin_bit_cast(typename Mma<T>::frag, vx);
 }
 
-// DMA of the 64 rows of a tile of two [N, 128] tensors (heads applied; the tile's first
-// row at byte r0b, its rows `pitch` bytes apart: the row pitch, or s times it when the
-// tile is gathered through the residue-s basis) into stage tiles at LDS m0 and m0 + kTB,
-// in four parts (instructions 2 part, 2 part + 1 of each tensor: with 4 waves each moves
-// two parts).  Wave w moves rows 32 w .. 32 w + 31; its instruction i writes rows
-// 32 w + 4 i + l / 16, lane l unit l % 16, fetching the unit the swizzle stores there:
-// (l % 16) ^ (4 (l / 16) + i % 4) (dvoff[i % 4]).
-__device__ __forceinline__ void dma_tile_part(uint32_t m0, const char* g0, const char* g1, int64_t pitch, int64_t r0b,
-                                              int w, const uint32_t* dvoff, int part) {
-  const char* a0 = g0 + r0b + 32 * w * pitch;
-  const char* a1 = g1 + r0b + 32 * w * pitch;
-  const uint32_t mw = m0 + (uint32_t)(32 * w * 256);
+// DMA of rows 16 w .. 16 w + 15 of a tile of two tensors (heads applied; the tile's first
+// row at byte r0b, its rows `pitch` bytes apart: the row pitch, or s times it when the tile
+// is gathered through the residue-s basis) into the stage at LDS m0.  Instruction i writes
+// rows 16 w + RPI i + l / UPR, lane l unit l % UPR, fetching the unit the swizzle stores
+// there (dvoff[i]).
+template <int D>
+__device__ __forceinline__ void dma_offsets(uint32_t* dvoff, int64_t pitch, int lane) {
+  const int r = lane / Tile<D>::UPR, u = lane % Tile<D>::UPR;
 #pragma unroll
-  for (int ii = 0; ii < 2; ++ii) {
-    const int i = 2 * part + ii;
-    dma_x4(mw + i * 1024, a0 + 4 * i * pitch, dvoff[i & 3]);
-    dma_x4(mw + kTB + i * 1024, a1 + 4 * i * pitch, dvoff[i & 3]);
+  for (int i = 0; i < Tile<D>::NI; ++i)
+    dvoff[i] = (uint32_t)(r * pitch) + 16u * (uint32_t)(u ^ Tile<D>::swz(Tile<D>::RPI * i + r));
+}
+template <int D>
+__device__ __forceinline__ void dma_tiles(uint32_t m0, const char* g0, const char* g1, int64_t pitch, int64_t r0b, int w,
+                                          const uint32_t* dvoff) {
+  const char* a0 = g0 + r0b + 16 * w * pitch;
+  const char* a1 = g1 + r0b + 16 * w * pitch;
+  const uint32_t mw = m0 + (uint32_t)(16 * w * Tile<D>::ROW);
+#pragma unroll
+  for (int i = 0; i < Tile<D>::NI; ++i) {
+    dma_x4(mw + i * 1024, a0 + Tile<D>::RPI * i * pitch, dvoff[i]);
+    dma_x4(mw + Tile<D>::TB + i * 1024, a1 + Tile<D>::RPI * i * pitch, dvoff[i]);
   }
 }
 
-// ---------------------------------------------------------------------------------
-// dK / dV (D = 128) with a key group's two products split over a pair of waves, so that
-// a wave holds half the state (one of K / V, one of dK / dV: about 200 registers) and
-// two waves share each SIMD.  Work-group: 4 waves, 64 keys; pair p owns keys
-// 32 p .. 32 p + 31.  Per tile (one listed query block, staged as in the kernels above):
-//   role 0: S = Q K^T, P = exp(scale S - lse) (masked), P to LDS; dV^T += dO^T P;
-//   role 1: dP = dO V^T; with P from LDS, dS = P (dP - rowsum(dO O)); dK^T += Q^T dS.
-// P goes through LDS in the MFMA operand layout (both roles map key m to lane m), as
-// 2-byte values: dS is formed from the rounded P that the MFMAs also use.
-constexpr int kPairP = kVecOff + 2 * kVec;          // P of both pairs: 2 x 4 KB
-constexpr int kPairTerms = kPairP + 2 * 4096;
-constexpr int kPairSmem = kPairTerms + PA_MAX_TERMS * (int)sizeof(pa_term);
+// Score elements dead in `word` (bit c of it = row or column c of the 32 the lane's
+// elements come from; element i is 8 (i / 4) + 4 G + i % 4) become 0.
+__device__ __forceinline__ void mask16(f32x16& p, uint32_t word, int G) {
+  const int32_t wv = (int32_t)(word >> (4 * G));
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const float pv = p[i];  // (a scalar copy: bit-casting the vector element itself reads element 0)
+    const int32_t keep = __builtin_amdgcn_sbfe(wv, 8 * (i >> 2) + (i & 3), 1);
+    p[i] = __builtin_bit_cast(float, __builtin_bit_cast(int32_t, pv) & keep);
+  }
+}
+
+// The lane's 32-bit word of live pairs of a partial tile without bitmaps: bit 8 (i / 4) +
+// 4 G + i % 4 set when pair i is live; q_at / k_at give the pair's original positions.
+template <typename QF, typename KF>
+__device__ __forceinline__ uint32_t live_word(const BwdK& a, const pa_term* terms, int G, QF q_at, KF k_at) {
+  uint32_t word = 0u;
+#pragma unroll 1
+  for (int i = 0; i < 16; ++i) {
+    const int b = 8 * (i >> 2) + 4 * G + (i & 3);
+    if (pred_live_rolled(terms, a.pred.n_include, a.pred.n_exclude, q_at(b), k_at(b), a.pred.dense_bits,
+                         a.pred.dense_words))
+      word |= 1u << b;
+  }
+  return word;
+}
+
+// A row's exponent offset -lse log2 e, -inf for a row with no live key (its P is then 0).
+__device__ __forceinline__ float neg_lse2(float lse) {
+  return lse == -INFINITY ? -INFINITY : -lse * 1.4426950408889634f;
+}
 
 template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_dkdv_pair_kernel(const BwdK a) {
-  using Frag = typename Mma<T>::frag;
-  constexpr int ESZ = 2, NKC = 8, NDB = 4;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char_t*)smem;
-  lds_cptr lds = (lds_cptr)smem;
-  pa_term* terms_s = reinterpret_cast<pa_term*>(smem + kPairTerms);
+__device__ __forceinline__ void to_frags(const f32x16& x, typename Mma<T>::frag* f) {
 #pragma unroll
-  for (int i = 0; i < PA_MAX_TERMS; ++i)  // (constant indices into the argument block)
-    if (threadIdx.x == i) terms_s[i] = a.pred.terms[i];
+  for (int c = 0; c < 2; ++c) {
+    f32x8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = x[8 * c + e];
+    f[c] = Mma<T>::cvt(v);
+  }
+}
+
+// The gradient rows of a work-group: each of its waves holds a partial X^T of one 32-row
+// half (half = the rows' half, part = which of the 2 NG partials), block db element
+// (i4, e) = column 32 db + 8 i4 + 4 G + e of row 32 half + m.  The partials go through LDS
+// (fp32, 16-byte units swizzled by row), are added, scaled, and leave as whole rows.
+// Thread t takes 8 columns of row (t + NT j) / (D / 8); with accumulate the stored rows are
+// loaded ahead (OldRows), so that their latency runs beside the last tile and the exchange.
+template <typename T, int D, int NG>
+struct OldRows {
+  static constexpr int NT = 256 * NG;
+  static constexpr int N = kBT * (D / 8) / NT;
+  typedef T t8 __attribute__((ext_vector_type(8)));
+  u32x4 x[N];
+  __device__ __forceinline__ static t8* at(const BwdK& a, char* head, int row0, int tid, int j) {
+    const int g = tid + NT * j, r = g / (D / 8), u = g % (D / 8);
+    return reinterpret_cast<t8*>(head + mem_row(a, row0 + r) * a.sn * 2 + 16 * u);
+  }
+  __device__ __forceinline__ void load(const BwdK& a, char* head, int row0, int tid) {
+    if (a.accumulate) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) x[j] = *reinterpret_cast<const u32x4*>(at(a, head, row0, tid, j));
+    }
+  }
+};
+template <typename T, int D, int NG>
+__device__ __forceinline__ void store_rows(const BwdK& a, char* smem, const f32x16* acc, int half, int part, int tid,
+                                           char* head, int row0, float scale, const OldRows<T, D, NG>& old) {
+  constexpr int NDB = D / 32, FU = D / 4;  // 16-byte units of a row of floats
+  using O = OldRows<T, D, NG>;
+  const int lane = tid & 63, G = lane >> 5, m = lane & 31;
+  lds_char_t* st = (lds_char_t*)smem;
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const f32x4 x = {acc[db][4 * i4], acc[db][4 * i4 + 1], acc[db][4 * i4 + 2], acc[db][4 * i4 + 3]};
+      *(lds_f4w*)(st + ((part * 2 + half) * 32 + m) * (D * 4) + 16 * ((8 * db + 2 * i4 + G) ^ (m & 15))) = x;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < O::N; ++j) {
+    const int g = tid + O::NT * j, r = g / (D / 8), u = g % (D / 8);
+    f32x8 x;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int at = r * (D * 4) + 16 * ((2 * u + k) ^ (r & 15));
+      f32x4 y = *(lds_f4*)(st + at);
+#pragma unroll
+      for (int pt = 1; pt < 2 * NG; ++pt) y += *(lds_f4*)(st + pt * kBT * FU * 16 + at);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[4 * k + e] = y[e] * scale;
+    }
+    if (a.accumulate) x += __builtin_convertvector(__builtin_bit_cast(typename O::t8, old.x[j]), f32x8);
+    *O::at(a, head, row0, tid, j) = __builtin_convertvector(x, typename O::t8);
+  }
+}
+
+// Issue position -> list position of a launch's n lists, longest first: every second run of
+// 32 goes backwards.  Work-groups are placed round-robin over an XCD's 32 CUs, so a CU whose
+// first list is among the longest of its run then takes the shortest of the next one.
+__device__ __forceinline__ int snake(int p, int n) {
+  const int r0 = p & ~31;
+  const int len = n - r0 < 32 ? n - r0 : 32;
+  return (p & 32) ? r0 + len - 1 - (p & 31) : p;
+}
+
+// ---------------------------------------------------------------------------------
+// dK / dV.  Work-group: 4 waves, one key block of 64; wave (kh, qh) takes keys 32 kh ..
+// +31 and, of every listed query block (a staged tile of Q and dO), rows 32 qh .. +31:
+//   S = Q K^T, P = exp(scale S - lse) (masked), dP = dO V^T, dS = P (dP - rowsum(dO O)),
+//   dV^T += dO^T P, dK^T += Q^T dS,
+// all on 32x32 MFMAs with the keys along the lanes, so P and dS are formed in the layout
+// the transposed products take them in: nothing passes between waves inside a tile, and
+// the one barrier per tile is the stage's.  The two query halves' partials are added
+// through LDS at the end.
+//
+// What bounds it: on long lists the MFMAs (causal, 32 heads x 8192, D = 128, bf16: both
+// kernels together 1.9 ms, 1.0 PFLOP/s of the 14 D per pair they issue, 80% of a large
+// torch matmul's rate); on short lists each item's start and end and its rows' bytes.  Two
+// waves per SIMD is what the registers allow at D = 128 (dK and dV take 128 of 256; K in
+// registers, V in LDS but for one fragment, address halves recomputed: 251 without spills).
+// Splitting a tile by quadrants replaced a pair of waves per 32 keys, one for P and dV and
+// one for dP and dK, that met at a barrier in the middle of every tile with P in LDS
+// (D = 128), and register-staged tiles that evaluated the mask and waited for each tile
+// (D = 64).  Measured: 32 heads x 16384 of band-256 | lattice-16 in bf16, D = 128, 1625 ->
+// 1260 us; causal, 8 heads x 4032 in f16, D = 64, 402 -> 100 us.
+//
+// NG groups of 4 waves share a work-group's list, group g taking tiles g, g + NG, ...; the
+// groups' partials are added with the halves'.  See launch_bwd for when.
+// The phases of a tile kept apart for the scheduler at D = 64 (108.6 -> 104 us of the causal
+// case above); at D = 128 it does better left alone (1302 -> 1289 us of the band and lattice).
+#define PA_FENCE() \
+  if constexpr (D == 64) __builtin_amdgcn_sched_barrier(0)
+template <int D>
+constexpr int v_in_regs() { return D == 64 ? 4 : 1; }  // V fragments kept in registers
+template <int D, int NG>
+constexpr int dkdv_smem() { return NG * Tile<D>::END + 2 * (D / 16 - v_in_regs<D>()) * 1024; }
+
+template <typename T, int D, bool BITS, int NG>
+__global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(D == 64 && NG == 1 ? 3 : 2)))
+void bwd_dkdv_kernel(const BwdK a) {
+  using Frag = typename Mma<T>::frag;
+  using TL = Tile<D>;
+  constexpr int ESZ = 2, NKC = D / 16, NDB = D / 32;
+  constexpr int NVR = v_in_regs<D>(), NVL = NKC - NVR;
+  extern __shared__ __attribute__((aligned(256))) char smem[];
+  pa_term* terms_s = reinterpret_cast<pa_term*>(smem + TL::TERMS_OFF);
+  if constexpr (!BITS) {
+#pragma unroll
+    for (int i = 0; i < PA_MAX_TERMS; ++i)  // (constant indices into the argument block)
+      if (threadIdx.x == i) terms_s[i] = a.pred.terms[i];
+  }
 
   const int tid = threadIdx.x, lane = tid & 63, G = lane >> 5, m = lane & 31;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int pair = w >> 1, role = w & 1;
+  const int wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = NG == 1 ? 0 : wg >> 2, w = wg & 3;
+  char* gsm = smem + grp * TL::END;  // this group's stages and vectors
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char_t*)gsm;
+  lds_cptr lds = (lds_cptr)gsm;
+  const int kh = w >> 1, qh = w & 1;
   const int64_t id = xcd_remap(blockIdx.x, (int64_t)gridDim.x);
-  const int kr = (int)(id % a.nb);
+  const int kr = snake((int)(id % a.nb), a.nb);
   const int kb = a.kv_order ? ((cint*)a.kv_order)[kr] : kr;
-  const int64_t bh = id / a.nb;
-  const int key = kb * kBT + pair * 32 + m;
+  const int64_t bh = gridDim.x / a.nb - 1 - id / a.nb;
+  const int key = kb * kBT + kh * 32 + m;
   const int key_o = orig_of(a.pred.perm_kv, key);
-  const int64_t key_m = mem_row(a, key);
   const int64_t rowb = a.sn * ESZ;
   const int rs = a.residue_s ? a.residue_s : 1;
   const int64_t pitch = rs * rowb;
   const char* hq = a.q + bh * a.sb * ESZ;
   const char* hdo = a.dout + bh * a.sb * ESZ;
-  const char* hlse = reinterpret_cast<const char*>(a.lse + bh * a.lse_sb);
+  const float* hlse = a.lse + bh * a.lse_sb;
   const char* hdvec = reinterpret_cast<const char*>(a.dvec + bh * a.lse_sb);
   const char* hperm = reinterpret_cast<const char*>(a.pred.perm_q);
-  const bool use_bits = a.q_bits != nullptr;
 
-  uint32_t dvoff[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    dvoff[j] = (uint32_t)((lane >> 4) * pitch) + 16u * (uint32_t)((lane & 15) ^ (4 * (lane >> 4) + j));
-  // query block qb into stage S: wave w moves rows 16 w .. 16 w + 15 of Q and dO; lse
-  // (and, without bitmaps, the original row numbers) by wave 0, rowsum(dO O) by wave 1,
-  // a partial tile's bitmap (bo >= 0) columns 32 (w - 2) .. +31 by waves 2 and 3
+  uint32_t dvoff[TL::NI];
+  dma_offsets<D>(dvoff, pitch, lane);
+  // Query block qb into stage S: the rows of Q and dO by every wave, rowsum(dO O) by wave 1,
+  // a partial tile's bitmap (bo >= 0) by waves 2 and 3 or, without bitmaps, the original row
+  // numbers by wave 2.  The lse goes through wave 0's registers (lse_n, written as the
+  // exponent offset by put_lse once it has arrived).
+  float lse_n = 0.f;
   auto dma = [&](int qb, int bo, int S) __attribute__((always_inline)) {
     const int64_t r0 = mem_row(a, qb * kBT);
-    dma_tile_part(lds0 + S * kStage, hq, hdo, pitch, r0 * rowb, pair, dvoff, 2 * role);
-    dma_tile_part(lds0 + S * kStage, hq, hdo, pitch, r0 * rowb, pair, dvoff, 2 * role + 1);
-    const uint32_t mv = lds0 + kVecOff + S * kVec;
-    if (w == 0) {
-      dma_x1(mv, hlse + r0 * 4, 4u * rs * lane);
-      if (hperm && !use_bits) dma_x1(mv + 512, hperm + (int64_t)qb * 256, 4u * lane);
-    } else if (w == 1) {
-      dma_x1(mv + 256, hdvec + r0 * 4, 4u * rs * lane);
-    } else if (use_bits && bo >= 0) {
-      dma_x1(mv + kBitsAt + 256 * (w - 2), reinterpret_cast<const char*>(a.q_bits + bo) + 256 * (w - 2), 4u * lane);
+    if (w == 0) lse_n = hlse[r0 + rs * lane];
+    dma_tiles<D>(lds0 + S * TL::STAGE, hq, hdo, pitch, r0 * rowb, w, dvoff);
+    const uint32_t mv = lds0 + TL::VEC_OFF + S * TL::VEC;
+    if (w == 1) dma_x1(mv + 256, hdvec + r0 * 4, 4u * rs * lane);
+    if constexpr (BITS) {
+      if (w >= 2 && bo >= 0)
+        dma_x1(mv + 512 + 256 * (w - 2), reinterpret_cast<const char*>(a.q_bits + bo) + 256 * (w - 2), 4u * lane);
+    } else if (hperm && w == 2) {
+      dma_x1(mv + 512, hperm + (int64_t)qb * 256, 4u * lane);
     }
   };
-
-  const TileReads rd = tile_reads(lds, lane);
-  lds_cptr vrow = lds + kVecOff + 16 * G;  // row vector entries 8 j + 4 G + 0..3 (+ 32 lb)
-  char* pbuf = smem + kPairP + pair * 4096 + lane * 16;  // this lane's P fragments (+ 1 KB per (lb, c))
-
-  // role 0 keeps K and dV, role 1 V and dK
-  Frag kv[NKC];
-  row_frags<T, 128>((role == 0 ? a.k : a.v) + (bh * a.sb + key_m * a.sn) * ESZ + 16 * G, kv);
-  f32x16 acc[NDB];
-#pragma unroll
-  for (int i = 0; i < NDB; ++i) acc[i] = f32x16{0};
-
-  // this lane's 16 x 2 score elements: element i of block lb is query row
-  // 32 lb + 8 (i / 4) + 4 G + i % 4, key `key`
-  auto scores = [&](int SO, int tile_off, f32x16* s) __attribute__((always_inline)) {
-#pragma unroll
-    for (int lb = 0; lb < 2; ++lb) {
-      u32x4 xa[NKC];
-#pragma unroll
-      for (int kc = 0; kc < NKC; ++kc) xa[kc] = *(lds_u4*)(rd.row[kc] + SO + tile_off + lb * 8192);
-      s[lb] = Mma<T>::mma(__builtin_bit_cast(Frag, xa[0]), kv[0], f32x16{0});
-#pragma unroll
-      for (int kc = 1; kc < NKC; ++kc) s[lb] = Mma<T>::mma(__builtin_bit_cast(Frag, xa[kc]), kv[kc], s[lb]);
-    }
+  auto put_lse = [&](int S) __attribute__((always_inline)) {
+    if (w == 0) *(lds_fw*)((lds_char_t*)gsm + TL::VEC_OFF + S * TL::VEC + 4 * lane) = neg_lse2(lse_n);
   };
-  // acc^T += X^T Y for the tile at tile_off (dO for dV, Q for dK), Y = the 4 fragments
-  auto accum = [&](int SO, int tile_off, const Frag* y) __attribute__((always_inline)) {
+
+  const TileReads<D> rd = tile_reads<D>(lds + 32 * qh * TL::ROW, lane);
+  lds_cptr vrow = lds + TL::VEC_OFF + 128 * qh + 16 * G;  // row vector entries 8 j + 4 G + 0..3
+
+  // K in registers; V partly in registers, the rest in LDS in fragment order (the
+  // accumulators of dK and dV already take half of a wave's registers).  Their rows come
+  // through stage 1, moved beside the first tile.
+  Frag kf[NKC], vf[NKC];
+  lds_char_t* vl = (lds_char_t*)smem + NG * TL::END + kh * NVL * 1024 + lane * 16;
+  f32x16 dkt[NDB], dvt[NDB];
 #pragma unroll
-    for (int lb = 0; lb < 2; ++lb) {
-      Frag fx[8];
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) fx[4 * c + db] = tr_frag_sw<T>(rd, db, SO + tile_off + (32 * lb + 16 * c) * 256);
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) acc[db] = Mma<T>::mma(fx[4 * c + db], y[2 * lb + c], acc[db]);
-    }
-  };
+  for (int i = 0; i < NDB; ++i) dkt[i] = dvt[i] = f32x16{0};
 
   auto tile = [&](auto SC, bool partial, int qb) __attribute__((always_inline)) {
     constexpr int S = decltype(SC)::value;
-    constexpr int SO = S * kStage;
-    if (role == 0) {
-      uint32_t live[2] = {0xffffu, 0xffffu};
-      if (partial && use_bits) {
-        const u32x2 bw = *(lds_u2*)(lds + kVecOff + S * kVec + kBitsAt + (32 * pair + m) * 8);
-        const uint32_t b0 = bw.x, b1 = bw.y;
-        live[0] = live16(b0, G);
-        live[1] = live16(b1, G);
-      } else if (partial) {
-        lds_i32* qo = (lds_i32*)(lds + kVecOff + S * kVec + 512);
+    constexpr int SO = S * TL::STAGE;
+    // element i of the lane: query row 32 qh + 8 (i / 4) + 4 G + i % 4, key `key`
+    f32x16 s = f32x16{0}, dp = f32x16{0};
 #pragma unroll
-        for (int lb = 0; lb < 2; ++lb) {
-          live[lb] = 0u;
-#pragma unroll 1
-          for (int i = 0; i < 16; ++i) {
-            const int qr = 32 * lb + 8 * (i >> 2) + 4 * G + (i & 3);
-            const int q_o = hperm ? qo[qr] : qb * kBT + qr;
-            if (pred_live_rolled(terms_s, a.pred.n_include, a.pred.n_exclude, q_o, key_o, a.pred.dense_bits,
-                                 a.pred.dense_words))
-              live[lb] |= 1u << i;
-          }
-        }
-      }
-      f32x4 l4[2][4];
+    for (int kc = 0; kc < NKC; ++kc)
+      s = Mma<T>::mma(__builtin_bit_cast(Frag, *(lds_u4*)(rd.row(kc) + SO)), kf[kc], s);
+    PA_FENCE();
 #pragma unroll
-      for (int lb = 0; lb < 2; ++lb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) l4[lb][j] = *(lds_f4*)(vrow + S * kVec + (32 * lb + 8 * j) * 4);
-      f32x16 s[2];
-      scores(SO, 0, s);
-      Frag pf[4];
-#pragma unroll
-      for (int lb = 0; lb < 2; ++lb)
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          f32x8 pv;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int i = 8 * c + e;
-            const float lse = l4[lb][i >> 2][i & 3];
-            const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(s[lb][i], a.c, -lse * 1.4426950408889634f));
-            pv[e] = (((live[lb] >> i) & 1u) && lse != -INFINITY) ? pe : 0.f;
-          }
-          pf[2 * lb + c] = Mma<T>::cvt(pv);
-          *reinterpret_cast<__attribute__((address_space(3))) u32x4*>((lds_char_t*)pbuf + (2 * lb + c) * 1024) =
-              __builtin_bit_cast(u32x4, pf[2 * lb + c]);
-        }
-      __syncthreads();  // P is in LDS
-      accum(SO, kTB, pf);  // dV^T += dO^T P
-    } else {
-      f32x4 d4[2][4];
-#pragma unroll
-      for (int lb = 0; lb < 2; ++lb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) d4[lb][j] = *(lds_f4*)(vrow + S * kVec + 256 + (32 * lb + 8 * j) * 4);
-      f32x16 dp[2];
-      scores(SO, kTB, dp);
-      __syncthreads();  // P is in LDS
-      Frag sf[4];
-#pragma unroll
-      for (int lb = 0; lb < 2; ++lb)
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const Frag pf = __builtin_bit_cast(Frag, *(lds_u4*)(lds + kPairP + pair * 4096 + lane * 16 + (2 * lb + c) * 1024));
-          const f32x8 pfl = __builtin_convertvector(pf, f32x8);
-          f32x8 sv;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const int i = 8 * c + e;
-            sv[e] = pfl[e] * (dp[lb][i] - d4[lb][i >> 2][i & 3]);
-          }
-          sf[2 * lb + c] = Mma<T>::cvt(sv);
-        }
-      accum(SO, 0, sf);  // dK^T += Q^T dS
+    for (int kc = 0; kc < NKC; ++kc) {
+      const Frag vx = kc < NVR ? vf[kc] : __builtin_bit_cast(Frag, *(lds_u4*)(vl + (kc - NVR) * 1024));
+      dp = Mma<T>::mma(__builtin_bit_cast(Frag, *(lds_u4*)(rd.row(kc) + SO + TL::TB)), vx, dp);
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 nl = *(lds_f4*)(vrow + S * TL::VEC + 32 * j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        s[4 * j + e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * j + e], a.c, nl[e]));
+    }
+    if (partial) {
+      uint32_t word;
+      if constexpr (BITS) {
+        word = *(lds_u32*)(lds + TL::VEC_OFF + S * TL::VEC + 512 + (32 * kh + m) * 8 + 4 * qh);
+      } else {
+        lds_i32* qo = (lds_i32*)(lds + TL::VEC_OFF + S * TL::VEC + 512 + 128 * qh);
+        word = live_word(a, terms_s, G, [&](int b) { return hperm ? qo[b] : qb * kBT + 32 * qh + b; },
+                         [&](int) { return key_o; });
+      }
+      mask16(s, word, G);
+    }
+    PA_FENCE();
+    Frag pf[2], sf[2];
+    to_frags<T>(s, pf);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+        dvt[db] = Mma<T>::mma(tr_frag<T, D>(rd, db, SO + TL::TB + 16 * c * TL::ROW), pf[c], dvt[db]);
+    PA_FENCE();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 dv = *(lds_f4*)(vrow + S * TL::VEC + 256 + 32 * j);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[4 * j + e] *= dp[4 * j + e] - dv[e];
+    }
+    to_frags<T>(s, sf);
+    PA_FENCE();
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+        dkt[db] = Mma<T>::mma(tr_frag<T, D>(rd, db, SO + 16 * c * TL::ROW), sf[c], dkt[db]);
   };
 
   const int nl = ((cint*)a.q_num)[kb];
   cint* qlist = (cint*)(a.q_idx + (int64_t)kb * a.tpitch);
   cbyte* plist = (cbyte*)(a.q_partial + (int64_t)kb * a.tpitch);
-  cint* olist = (cint*)(use_bits ? a.q_bits_off + (int64_t)kb * a.tpitch : a.q_idx);
+  cint* olist = (cint*)(BITS ? a.q_bits_off + (int64_t)kb * a.tpitch : a.q_idx);
   auto tile_of = [&](int t, int& qb, int& bo) __attribute__((always_inline)) {
     qb = qlist[t];
-    bo = use_bits ? olist[t] : (plist[t] != 0 ? 0 : -1);
+    bo = BITS ? olist[t] : (plist[t] != 0 ? 0 : -1);
   };
   int qb_c = 0, bo_c = -1, qb_n = 0, bo_n = -1;
   if (nl > 0) {
-    tile_of(0, qb_c, bo_c);
-    dma(qb_c, bo_c, 0);
+    if (grp < nl) {
+      tile_of(grp, qb_c, bo_c);
+      dma(qb_c, bo_c, 0);
+    }
+    dma_tiles<D>(lds0 + TL::STAGE, a.k + bh * a.sb * ESZ, a.v + bh * a.sb * ESZ, pitch, mem_row(a, kb * kBT) * rowb, w,
+                 dvoff);
+    put_lse(0);
+    if (NG + grp < nl) tile_of(NG + grp, qb_n, bo_n);
+    dma_wait_all();
+    __syncthreads();
+    const TileReads<D> kd = tile_reads<D>(lds + TL::STAGE + 32 * kh * TL::ROW, lane);
+#pragma unroll
+    for (int kc = 0; kc < NKC; ++kc) {
+      kf[kc] = __builtin_bit_cast(Frag, *(lds_u4*)(kd.row(kc)));
+      vf[kc] = __builtin_bit_cast(Frag, *(lds_u4*)(kd.row(kc) + TL::TB));
+    }
+    if (grp == 0 && qh == 0) {
+#pragma unroll
+      for (int kc = NVR; kc < NKC; ++kc) *(lds_u4w*)(vl + (kc - NVR) * 1024) = __builtin_bit_cast(u32x4, vf[kc]);
+    }
   }
-  if (nl > 1) tile_of(1, qb_n, bo_n);
   auto step = [&](auto SC, int t) __attribute__((always_inline)) {
     constexpr int S = decltype(SC)::value;
     dma_wait_all();
-    __syncthreads();  // stage S is in; every wave is past stage S ^ 1 and the last P
-    if (t + 1 < nl) dma(qb_n, bo_n, S ^ 1);
+    __syncthreads();  // stage S is in; every wave is past stage S ^ 1
+    if (t + NG < nl) dma(qb_n, bo_n, S ^ 1);
     const int qb = qb_c;
     const bool partial = bo_c >= 0;
     qb_c = qb_n;
     bo_c = bo_n;
-    if (t + 2 < nl) tile_of(t + 2, qb_n, bo_n);
-    tile(SC, partial, qb);
+    if (t + 2 * NG < nl) tile_of(t + 2 * NG, qb_n, bo_n);
+    if (NG == 1 || t < nl) tile(SC, partial, qb);
+    if (t + NG < nl) put_lse(S ^ 1);
   };
+  // (every group takes every step: the last one may have no tile for it)
+  const int ns = (nl + NG - 1) / NG;
   int t = 0;
-  for (; t + 1 < nl; t += 2) {
-    step(std::integral_constant<int, 0>{}, t);
-    step(std::integral_constant<int, 1>{}, t + 1);
+  for (; t + 1 < ns; t += 2) {
+    step(std::integral_constant<int, 0>{}, t * NG + grp);
+    step(std::integral_constant<int, 1>{}, (t + 1) * NG + grp);
   }
-  if (t < nl) step(std::integral_constant<int, 0>{}, t);
+  if (t < ns) step(std::integral_constant<int, 0>{}, t * NG + grp);
 
-  // role 0: dV^T, role 1: dK^T blocks [32 d x 32 keys]: lane (key m, G) holds
-  // d = 32 db + 8 i4 + 4 G + 0..3
-  char* grow = (role == 0 ? a.dv : a.dk) + (bh * a.sb + key_m * a.sn) * ESZ;
-  const float gs = role == 0 ? 1.f : a.scale;
-#pragma unroll
-  for (int db = 0; db < NDB; ++db) {
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const int d0 = 32 * db + 8 * i4 + 4 * G;
-      f32x4 x = {acc[db][4 * i4], acc[db][4 * i4 + 1], acc[db][4 * i4 + 2], acc[db][4 * i4 + 3]};
-      x *= gs;
-      store_grad4<T>(grow + d0 * ESZ, x, a.accumulate);
-    }
-  }
+  char* hdv = a.dv + bh * a.sb * ESZ;
+  char* hdk = a.dk + bh * a.sb * ESZ;
+  OldRows<T, D, NG> odv, odk;
+  odv.load(a, hdv, kb * kBT, tid);
+  odk.load(a, hdk, kb * kBT, tid);
+  __syncthreads();  // every wave is past its tiles
+  store_rows<T, D, NG>(a, smem, dvt, kh, 2 * grp + qh, tid, hdv, kb * kBT, 1.f, odv);
+  __syncthreads();
+  store_rows<T, D, NG>(a, smem, dkt, kh, 2 * grp + qh, tid, hdk, kb * kBT, a.scale, odk);
 }
 
-template <typename T>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) void bwd_dq_stream_kernel(const BwdK a) {
+// ---------------------------------------------------------------------------------
+// dQ, the same with the roles of queries and keys exchanged (the forward's layout): wave
+// (qh, kh) takes query rows 32 qh .. +31 of the work-group's block and, of every listed key
+// block (a staged tile of K and V), keys 32 kh .. +31:
+//   S^T = K Q^T, dP^T = V dO^T, dQ^T += K^T dS^T,
+// with the queries along the lanes; the two key halves' partials are added at the end.
+template <typename T, int D, bool BITS, int NG>
+__global__ __launch_bounds__(256 * NG) __attribute__((amdgpu_waves_per_eu(D == 64 && NG == 1 ? 3 : 2)))
+void bwd_dq_kernel(const BwdK a) {
   using Frag = typename Mma<T>::frag;
-  constexpr int ESZ = 2, NKC = 8, NDB = 4;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char_t*)smem;
-  lds_cptr lds = (lds_cptr)smem;
-  pa_term* terms_s = reinterpret_cast<pa_term*>(smem + kTermsOff);
+  using TL = Tile<D>;
+  constexpr int ESZ = 2, NKC = D / 16, NDB = D / 32;
+  extern __shared__ __attribute__((aligned(256))) char smem[];
+  pa_term* terms_s = reinterpret_cast<pa_term*>(smem + TL::TERMS_OFF);
+  if constexpr (!BITS) {
 #pragma unroll
-  for (int i = 0; i < PA_MAX_TERMS; ++i)
-    if (threadIdx.x == i) terms_s[i] = a.pred.terms[i];
+    for (int i = 0; i < PA_MAX_TERMS; ++i)
+      if (threadIdx.x == i) terms_s[i] = a.pred.terms[i];
+  }
 
   const int tid = threadIdx.x, lane = tid & 63, G = lane >> 5, m = lane & 31;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = NG == 1 ? 0 : wg >> 2, w = wg & 3;
+  char* gsm = smem + grp * TL::END;  // this group's stages and vectors
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_char_t*)gsm;
+  lds_cptr lds = (lds_cptr)gsm;
+  const int qh = w >> 1, kh = w & 1;
   const int64_t id = xcd_remap(blockIdx.x, (int64_t)gridDim.x);
-  const int qb = (int)(id % a.nb);
+  // the last query blocks first: a causal mask's lists grow along the sequence, and the
+  // longest should not be the last to start
+  const int qb = a.nb - 1 - snake((int)(id % a.nb), a.nb);
   const int64_t bh = id / a.nb;
-  const int row = qb * kBT + w * 32 + m;  // this lane's query row (index space)
+  const int row = qb * kBT + qh * 32 + m;  // this lane's query row (index space)
   const int q_o = orig_of(a.pred.perm_q, row);
   const int64_t row_m = mem_row(a, row);
   const int64_t rowb = a.sn * ESZ;
@@ -729,202 +591,117 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const char* hv = a.v + bh * a.sb * ESZ;
   const char* hperm = reinterpret_cast<const char*>(a.pred.perm_kv);
 
-  uint32_t dvoff[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    dvoff[j] = (uint32_t)((lane >> 4) * pitch) + 16u * (uint32_t)((lane & 15) ^ (4 * (lane >> 4) + j));
-  const bool use_bits = a.kv_bits != nullptr;
-  // key block kb into stage S: K and V tiles; without bitmaps the original key numbers by
-  // wave 0; a partial tile's bitmap (bo >= 0), rows 32 w .. 32 w + 31 by wave w
-  auto dma = [&](int kb, int bo, int S, int part) __attribute__((always_inline)) {
-    dma_tile_part(lds0 + S * kStage, hk, hv, pitch, mem_row(a, kb * kBT) * rowb, w, dvoff, part);
-    if (part) return;
-    const uint32_t mv = lds0 + kVecOff + S * kVec;
-    if (hperm && !use_bits && w == 0) dma_x1(mv + 512, hperm + (int64_t)kb * 256, 4u * lane);
-    if (use_bits && bo >= 0)
-      dma_x1(mv + kBitsAt + 256 * w, reinterpret_cast<const char*>(a.kv_bits + bo) + 256 * w, 4u * lane);
+  uint32_t dvoff[TL::NI];
+  dma_offsets<D>(dvoff, pitch, lane);
+  // key block kb into stage S: the rows of K and V by every wave, a partial tile's bitmap
+  // (bo >= 0) by waves 0 and 1 or, without bitmaps, the original key numbers by wave 0
+  auto dma = [&](int kb, int bo, int S) __attribute__((always_inline)) {
+    dma_tiles<D>(lds0 + S * TL::STAGE, hk, hv, pitch, mem_row(a, kb * kBT) * rowb, w, dvoff);
+    const uint32_t mv = lds0 + TL::VEC_OFF + S * TL::VEC + 512;
+    if constexpr (BITS) {
+      if (w < 2 && bo >= 0) dma_x1(mv + 256 * w, reinterpret_cast<const char*>(a.kv_bits + bo) + 256 * w, 4u * lane);
+    } else if (hperm && w == 0) {
+      dma_x1(mv, hperm + (int64_t)kb * 256, 4u * lane);
+    }
   };
 
-  const TileReads rd = tile_reads(lds, lane);
+  const TileReads<D> rd = tile_reads<D>(lds + 32 * kh * TL::ROW, lane);
 
+  // Q and dO in registers: their rows come through stage 1, moved beside the first tile
   Frag qf[NKC], df[NKC];
-  row_frags<T, 128>(a.q + (bh * a.sb + row_m * a.sn) * ESZ + 16 * G, qf);
-  row_frags<T, 128>(a.dout + (bh * a.sb + row_m * a.sn) * ESZ + 16 * G, df);
-  const float lse = a.lse[bh * a.lse_sb + row_m];
-  const float nl2 = -lse * 1.4426950408889634f;
-  const bool dead = lse == -INFINITY;
+  const float nl2 = neg_lse2(a.lse[bh * a.lse_sb + row_m]);
   const float dr = a.dvec[bh * a.lse_sb + row_m];
   f32x16 dqt[NDB];
 #pragma unroll
   for (int i = 0; i < NDB; ++i) dqt[i] = f32x16{0};
 
-  // One tile (stage S), phases as in the dK/dV kernel: A scores of keys 0..31; B scores of
-  // keys 32..63 beside the gradient of keys 0..31; C dQ^T += K^T dS^T of keys 0..31 beside
-  // the gradient of 32..63; D dQ^T of keys 32..63.  Element i of a score block is key
-  // 32 lb + 8 (i / 4) + 4 G + i % 4, query `row`.
-  auto compute = [&](auto SC, bool partial, int kb, auto&& pre) __attribute__((always_inline)) {
+  auto tile = [&](auto SC, bool partial, int kb) __attribute__((always_inline)) {
     constexpr int S = decltype(SC)::value;
-    constexpr int SO = S * kStage;
-    uint32_t live[2] = {dead ? 0u : 0xffffu, dead ? 0u : 0xffffu};
-    if (partial && !dead && use_bits) {
-      // this lane's row of the tile: columns 0..31, 32..63
-      const u32x2 bw = *(lds_u2*)(lds + kVecOff + S * kVec + kBitsAt + (32 * w + m) * 8);
-      const uint32_t b0 = bw.x, b1 = bw.y;
-      live[0] = live16(b0, G);
-      live[1] = live16(b1, G);
-    } else if (partial && !dead) {
-      lds_i32* ko = (lds_i32*)(lds + kVecOff + S * kVec + 512);
+    constexpr int SO = S * TL::STAGE;
+    // element i of the lane: key 32 kh + 8 (i / 4) + 4 G + i % 4, query `row`
+    f32x16 s = f32x16{0}, dp = f32x16{0};
 #pragma unroll
-      for (int lb = 0; lb < 2; ++lb) {
-        live[lb] = 0u;
-#pragma unroll 1
-        for (int i = 0; i < 16; ++i) {
-          const int kr = 32 * lb + 8 * (i >> 2) + 4 * G + (i & 3);
-          const int k_o = hperm ? ko[kr] : kb * kBT + kr;
-          if (pred_live_rolled(terms_s, a.pred.n_include, a.pred.n_exclude, q_o, k_o, a.pred.dense_bits,
-                               a.pred.dense_words))
-            live[lb] |= 1u << i;
-        }
+    for (int kc = 0; kc < NKC; ++kc)
+      s = Mma<T>::mma(__builtin_bit_cast(Frag, *(lds_u4*)(rd.row(kc) + SO)), qf[kc], s);
+#pragma unroll
+    for (int kc = 0; kc < NKC; ++kc)
+      dp = Mma<T>::mma(__builtin_bit_cast(Frag, *(lds_u4*)(rd.row(kc) + SO + TL::TB)), df[kc], dp);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.c, nl2));
+    if (partial) {
+      uint32_t word;
+      if constexpr (BITS) {
+        word = *(lds_u32*)(lds + TL::VEC_OFF + S * TL::VEC + 512 + (32 * qh + m) * 8 + 4 * kh);
+      } else {
+        lds_i32* ko = (lds_i32*)(lds + TL::VEC_OFF + S * TL::VEC + 512 + 128 * kh);
+        word = live_word(a, terms_s, G, [&](int) { return q_o; },
+                         [&](int b) { return hperm ? ko[b] : kb * kBT + 32 * kh + b; });
       }
-    }
-    auto scores = [&](int lb, f32x16& s, f32x16& dp) __attribute__((always_inline)) {
-      u32x4 ka[NKC], va[NKC];
-#pragma unroll
-      for (int kc = 0; kc < NKC; ++kc) {
-        ka[kc] = *(lds_u4*)(rd.row[kc] + SO + lb * 8192);
-        va[kc] = *(lds_u4*)(rd.row[kc] + SO + kTB + lb * 8192);
-      }
-      s = Mma<T>::mma(__builtin_bit_cast(Frag, ka[0]), qf[0], f32x16{0});
-      dp = Mma<T>::mma(__builtin_bit_cast(Frag, va[0]), df[0], f32x16{0});
-#pragma unroll
-      for (int kc = 1; kc < NKC; ++kc) {
-        s = Mma<T>::mma(__builtin_bit_cast(Frag, ka[kc]), qf[kc], s);
-        dp = Mma<T>::mma(__builtin_bit_cast(Frag, va[kc]), df[kc], dp);
-      }
-    };
-    auto grads = [&](int lb, const f32x16& s, const f32x16& dp, Frag* sf) __attribute__((always_inline)) {
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        f32x8 sv;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int i = 8 * c + e;
-          const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.c, nl2));
-          const float p = ((live[lb] >> i) & 1u) ? pe : 0.f;
-          sv[e] = p * (dp[i] - dr);
-        }
-        sf[c] = Mma<T>::cvt(sv);
-      }
-    };
-    // dQ^T += K^T dS^T for keys 32 lb .. +31: the transposed K fragments (chunk c, block db
-    // at 4 c + db) are read first, into registers
-    auto tr_reads = [&](int lb, Frag* fk) __attribute__((always_inline)) {
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const int off = SO + (32 * lb + 16 * c) * 256;
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) fk[4 * c + db] = tr_frag_sw<T>(rd, db, off);
-      }
-    };
-    auto accum = [&](const Frag* fk, const Frag* sf) __attribute__((always_inline)) {
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) dqt[db] = Mma<T>::mma(fk[4 * c + db], sf[c], dqt[db]);
-    };
-    f32x16 s0, dp0, s1, dp1;
-    Frag sf0[2], sf1[2], fk[8];
-    pre(0);
-    pre(1);
-    pre(2);
-    pre(3);
-    scores(0, s0, dp0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-    for (int q_ = 0; q_ < 12; ++q_) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    scores(1, s1, dp1);
-    grads(0, s0, dp0, sf0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-    for (int q_ = 0; q_ < 12; ++q_) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+      mask16(s, word, G);
     }
 #pragma unroll
-    for (int q_ = 0; q_ < 4; ++q_) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    tr_reads(0, fk);
-    grads(1, s1, dp1, sf1);
-    accum(fk, sf0);
-    __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);
+    for (int i = 0; i < 16; ++i) s[i] *= dp[i] - dr;
+    Frag sf[2];
+    to_frags<T>(s, sf);
 #pragma unroll
-    for (int q_ = 0; q_ < 8; ++q_) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    tr_reads(1, fk);
-    accum(fk, sf1);
-    __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);
-    __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+        dqt[db] = Mma<T>::mma(tr_frag<T, D>(rd, db, SO + 16 * c * TL::ROW), sf[c], dqt[db]);
   };
 
   const int nl = ((cint*)a.kv_num)[qb];
   cint* klist = (cint*)(a.kv_idx + (int64_t)qb * a.pitch);
   cbyte* plist = (cbyte*)(a.kv_partial + (int64_t)qb * a.pitch);
-  cint* olist = (cint*)(use_bits ? a.kv_bits_off + (int64_t)qb * a.pitch : a.kv_idx);
+  cint* olist = (cint*)(BITS ? a.kv_bits_off + (int64_t)qb * a.pitch : a.kv_idx);
   auto tile_of = [&](int t, int& kb, int& bo) __attribute__((always_inline)) {
     kb = klist[t];
-    bo = use_bits ? olist[t] : (plist[t] != 0 ? 0 : -1);
+    bo = BITS ? olist[t] : (plist[t] != 0 ? 0 : -1);
   };
   int kb_c = 0, bo_c = -1, kb_n = 0, bo_n = -1;
   if (nl > 0) {
-    tile_of(0, kb_c, bo_c);
+    if (grp < nl) {
+      tile_of(grp, kb_c, bo_c);
+      dma(kb_c, bo_c, 0);
+    }
+    dma_tiles<D>(lds0 + TL::STAGE, a.q + bh * a.sb * ESZ, a.dout + bh * a.sb * ESZ, pitch, mem_row(a, qb * kBT) * rowb, w,
+                 dvoff);
+    if (NG + grp < nl) tile_of(NG + grp, kb_n, bo_n);
+    dma_wait_all();
+    __syncthreads();
+    const TileReads<D> qd = tile_reads<D>(lds + TL::STAGE + 32 * qh * TL::ROW, lane);
 #pragma unroll
-    for (int part = 0; part < 4; ++part) dma(kb_c, bo_c, 0, part);
+    for (int kc = 0; kc < NKC; ++kc) {
+      qf[kc] = __builtin_bit_cast(Frag, *(lds_u4*)(qd.row(kc)));
+      df[kc] = __builtin_bit_cast(Frag, *(lds_u4*)(qd.row(kc) + TL::TB));
+    }
   }
-  if (nl > 1) tile_of(1, kb_n, bo_n);
   auto step = [&](auto SC, int t) __attribute__((always_inline)) {
     constexpr int S = decltype(SC)::value;
     dma_wait_all();
     __syncthreads();
-    const bool more = t + 1 < nl;
-    const int kb = kb_c, kb_d = kb_n, bo_d = bo_n;
+    if (t + NG < nl) dma(kb_n, bo_n, S ^ 1);
+    const int kb = kb_c;
     const bool partial = bo_c >= 0;
     kb_c = kb_n;
     bo_c = bo_n;
-    if (t + 2 < nl) tile_of(t + 2, kb_n, bo_n);
-    compute(SC, partial, kb, [&](int part) __attribute__((always_inline)) {
-      if (more) dma(kb_d, bo_d, S ^ 1, part);
-    });
+    if (t + 2 * NG < nl) tile_of(t + 2 * NG, kb_n, bo_n);
+    if (NG == 1 || t < nl) tile(SC, partial, kb);
   };
+  // (every group takes every step: the last one may have no tile for it)
+  const int ns = (nl + NG - 1) / NG;
   int t = 0;
-  for (; t + 1 < nl; t += 2) {
-    step(std::integral_constant<int, 0>{}, t);
-    step(std::integral_constant<int, 1>{}, t + 1);
+  for (; t + 1 < ns; t += 2) {
+    step(std::integral_constant<int, 0>{}, t * NG + grp);
+    step(std::integral_constant<int, 1>{}, (t + 1) * NG + grp);
   }
-  if (t < nl) step(std::integral_constant<int, 0>{}, t);
+  if (t < ns) step(std::integral_constant<int, 0>{}, t * NG + grp);
 
-  char* dqrow = a.dq + (bh * a.sb + row_m * a.sn) * ESZ;
-#pragma unroll
-  for (int db = 0; db < NDB; ++db) {
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const int d0 = 32 * db + 8 * i4 + 4 * G;
-      f32x4 x = {dqt[db][4 * i4], dqt[db][4 * i4 + 1], dqt[db][4 * i4 + 2], dqt[db][4 * i4 + 3]};
-      x *= a.scale;
-      store_grad4<T>(dqrow + d0 * ESZ, x, a.accumulate);
-    }
-  }
+  char* hdq = a.dq + bh * a.sb * ESZ;
+  OldRows<T, D, NG> odq;
+  odq.load(a, hdq, qb * kBT, tid);
+  __syncthreads();  // every wave is past its tiles
+  store_rows<T, D, NG>(a, smem, dqt, qh, 2 * grp + kh, tid, hdq, qb * kBT, a.scale, odq);
 }
 
 // Transposed block lists: for key block kb, the query blocks whose list holds kb, in
@@ -974,6 +751,36 @@ __global__ __launch_bounds__(64) void bits_transpose_kernel(const int32_t* kv_bi
   q_bits[off + 2 * k + 1] = col[1];
 }
 
+template <typename T, int D, bool BITS, int NG>
+int launch_bwd_t(const BwdK& k, int64_t BH, hipStream_t s) {
+  constexpr int kv_smem = dkdv_smem<D, NG>(), q_smem = NG * Tile<D>::END;
+  // the dynamic LDS limit is raised once per device
+  static unsigned long long configured = 0ull;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
+  if (dev >= 64 || !((configured >> dev) & 1ull)) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dkdv_kernel<T, D, BITS, NG>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kv_smem);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dq_kernel<T, D, BITS, NG>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, q_smem);
+    if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(bwd kernels)");
+    if (dev < 64) configured |= 1ull << dev;
+  }
+  const unsigned grid = (unsigned)(k.nb * BH);
+  hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, BITS, NG>), dim3(grid), dim3(256 * NG), kv_smem, s, k);
+  PA_LAUNCH_CHECK("bwd_dkdv_kernel");
+  hipLaunchKernelGGL((bwd_dq_kernel<T, D, BITS, NG>), dim3(grid), dim3(256 * NG), q_smem, s, k);
+  PA_LAUNCH_CHECK("bwd_dq_kernel");
+  return PA_OK;
+}
+
+// Two groups of waves per list where one would leave the chip waiting for its longest
+// lists: a work-group for every CU or fewer, or up to two with a list of 32 tiles or more.
+// One group / two, both kernels and the pre-pass, causal f16 D = 64: 64 work-groups (longest
+// list 32) 54.0 / 39.3 us, 504 (63) 107.6 / 101.4 us; window 512, bf16, 448 work-groups
+// (9): 33.5 / 38.8 us; causal, 1024 work-groups (64): 162.6 / 179.4 us.
 template <typename T, int D>
 int launch_bwd(const BwdK& k, int64_t BH, bool dvec_given, hipStream_t s) {
   const int64_t rows = BH * k.N;
@@ -982,33 +789,10 @@ int launch_bwd(const BwdK& k, int64_t BH, bool dvec_given, hipStream_t s) {
                        rows);
     PA_LAUNCH_CHECK("bwd_pre_kernel");
   }
-  if constexpr (D == 128) {
-    // the dynamic LDS limit is raised once per device
-    static unsigned long long configured = 0ull;
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
-    if (dev >= 64 || !((configured >> dev) & 1ull)) {
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dkdv_pair_kernel<T>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, kPairSmem);
-      if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_dq_stream_kernel<T>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kBwdSmem);
-      if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(bwd stream kernels)");
-      if (dev < 64) configured |= 1ull << dev;
-    }
-    const unsigned grid = (unsigned)(k.nb * BH);
-    hipLaunchKernelGGL(bwd_dkdv_pair_kernel<T>, dim3(grid), dim3(256), kPairSmem, s, k);
-    PA_LAUNCH_CHECK("bwd_dkdv_pair_kernel");
-    hipLaunchKernelGGL(bwd_dq_stream_kernel<T>, dim3(grid), dim3(128), kBwdSmem, s, k);
-    PA_LAUNCH_CHECK("bwd_dq_stream_kernel");
-  } else {
-    hipLaunchKernelGGL((bwd_dkdv_kernel<T, D>), dim3((unsigned)k.nb, (unsigned)BH), dim3(128), 0, s, k);
-    PA_LAUNCH_CHECK("bwd_dkdv_kernel");
-    hipLaunchKernelGGL((bwd_dq_kernel<T, D>), dim3((unsigned)k.nb, (unsigned)BH), dim3(128), 0, s, k);
-    PA_LAUNCH_CHECK("bwd_dq_kernel");
-  }
-  return PA_OK;
+  if (!k.q_bits) return launch_bwd_t<T, D, false, 1>(k, BH, s);
+  const int64_t grid = k.nb * BH, longest = k.tpitch > k.pitch ? k.tpitch : k.pitch;
+  const bool two = grid <= 256 || (grid <= 512 && longest >= 32);
+  return two ? launch_bwd_t<T, D, true, 2>(k, BH, s) : launch_bwd_t<T, D, true, 1>(k, BH, s);
 }
 
 }  // namespace

@@ -67,6 +67,33 @@ def _gradients_case(gpu, name, dtype, D, bitmaps):
     _check(grads, want, dtype, f"{name} {dtype} D={D} bitmaps={bitmaps}")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("name,BH,N", [
+    ("causal", 1, 64), ("causal", 1, 192),            # lists of 1 to 3 tiles: two groups of waves, odd ends
+    ("causal", 4, 4096), ("causal", 5, 4160),         # 256 and 325 work-groups, lists up to 64 and 65: two groups
+    ("window-128", 8, 2112),                          # 264 work-groups, lists of 3: one group
+    ("causal", 31, 1088),                             # 527 work-groups: one group, lists of 1 to 17
+])
+def test_gradients_at_the_group_rule(gpu, name, BH, N, D):
+    """Both sides of the rule that gives a list two groups of waves (at most 256 work-groups,
+    or at most 512 and a list of 32 tiles), overwriting and then accumulating, against the
+    oracle on the last head."""
+    q, k, v = make_qkv(BH, N, D, torch.float16, seed=N + D)
+    do = make_qkv(BH, N, D, torch.float16, seed=N + D + 1)[0]
+    rows = oatt.spec_rows(om.NAMED[name], N)
+    dev = [x.to(gpu) for x in (q, k, v)]
+    lse = torch.empty(BH, N, device=gpu)
+    bi = pindex.build(numpy_mask(name), N, 64, 64)
+    o = pattn.block_sparse_attention(*dev, *pindex.to_cuda(bi, gpu), *triton_params(name), 64, 64, lse=lse)
+    plan = pbwd.BackwardPlan(numpy_mask(name), N, gpu)
+    grads = plan.backward(*dev, o, lse, do.to(gpu))
+    _, _, want = _oracle(*(x[-1:] for x in (q, k, v, do)), rows)
+    _check([g[-1:] for g in grads], want, torch.float16, f"{name} BH={BH} N={N} D={D}")
+    twice = plan.backward(*dev, o, lse, do.to(gpu), dq=grads[0].clone(), dk=grads[1].clone(), dv=grads[2].clone(),
+                          accumulate=True)
+    _check([g[-1:] for g in twice], [2 * x for x in want], torch.float16, f"accumulate {name} BH={BH} N={N} D={D}")
+
+
 def test_forward_then_backward(gpu):
     """The streaming forward's o and lse feed the backward."""
     BH, N, D, name = 2, 2048, 128, "band256+lat16"
