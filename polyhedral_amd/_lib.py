@@ -94,6 +94,7 @@ SIGNATURES = {
     "pa_invert_perm": (ctypes.c_int, [c_vp, c_vp, c_i64, c_vp]),
     "pa_residue_perm": (ctypes.c_int, [c_vp, c_i64, c_i32, c_vp]),
     "pa_attn_fwd": (ctypes.c_int, [ctypes.POINTER(PaAttnArgs), c_vp]),
+    "pa_attn_fwd_tile": (ctypes.c_int, [ctypes.POINTER(PaAttnArgs), c_vp]),
     "pa_lse_merge": (ctypes.c_int, [ctypes.POINTER(c_vp), ctypes.POINTER(c_vp), c_i32, c_vp, c_i32, c_vp,
                                     c_i64, c_i64, c_i32, c_vp]),
     "pa_kv_append": (ctypes.c_int, [c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_i64, c_i32, c_i32,

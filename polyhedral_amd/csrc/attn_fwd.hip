@@ -9,6 +9,8 @@ int launch_attn_bf16(const AttnK& a, int D, int NW, hipStream_t s);
 int launch_attn_f16(const AttnK& a, int D, int NW, hipStream_t s);
 int launch_attn_f32(const AttnK& a, int D, int NW, hipStream_t s);
 int launch_attn_wsplit(const AttnK& a, int D, hipStream_t s);
+bool attn_tile_takes(const AttnK& a, int dtype);
+int launch_attn_tile(const AttnK& a, int dtype, int D, hipStream_t s);
 int launch_attn_stream(const AttnK& a, int dtype, hipStream_t s);
 int launch_attn_run(const AttnK& a, int groups, int dtype, bool cooperative, hipStream_t s);
 int launch_attn_split_grid(const AttnK& a, int dtype, hipStream_t s);
@@ -194,6 +196,18 @@ extern "C" int pa_attn_fwd(const pa_attn_args* x, void* stream) {
     case PA_F16: return pa::launch_attn_f16(a, x->D, NW, s);
     default: return pa::launch_attn_f32(a, x->D, NW, s);
   }
+}
+
+extern "C" int pa_attn_fwd_tile(const pa_attn_args* x, void* stream) {
+  pa::AttnK a;
+  if (int rc = pa::fill_attn(x, a)) return rc;
+  PA_CHECK_ARG(x->run_groups == 0 && !x->wave_split && !x->kv_steps,
+               "pa_attn_fwd_tile: takes no run_groups, wave_split or kv_steps");
+  PA_CHECK_ARG(pa::attn_tile_takes(a, x->dtype),
+               "pa_attn_fwd_tile: needs f16 or bf16, BQ = 64 or 128, no K / V gather through a table and no class-B "
+               "emulation (dtype %d, BQ %d)",
+               x->dtype, x->BQ);
+  return pa::launch_attn_tile(a, x->dtype, x->D, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int pa_attn_fwd_split(const pa_split_args* x, void* stream) {

@@ -19,7 +19,7 @@
 
 #include <type_traits>
 
-#include "attn_kernel.hpp"
+#include "lds_rows.hpp"
 
 namespace pa {
 namespace {
@@ -98,111 +98,29 @@ __device__ __forceinline__ int32_t orig_of(const int32_t* perm, int32_t r) { ret
 
 // ---- staged tiles ------------------------------------------------------------------
 // A tile of 64 rows of two tensors is brought into LDS by LDS DMA (no staging registers,
-// no LDS stores), two stages deep: the next listed tile moves while the current one is
-// consumed, behind one wait and one barrier per tile.  A DMA instruction writes 64
-// consecutive 16-byte units, so the rows are stored unpadded and one XOR swizzle of the
-// 16-byte units serves both ways a tile is read (unit u of row r sits at u ^ swz(r)):
-//  * D = 128 (256-byte rows): 4 (r % 4) + (r / 4) % 4.  The 16 rows of a 16-byte row read
-//    land on 16 different units of the 256-byte bank window, and the 4 rows of a transposed
-//    read on 4 different 64-byte groups;
-//  * D = 64 (128-byte rows, two to a bank window): with x = (r / 2) % 8, 4 (x % 2) + x / 2.
-//    The 8 row pairs of a row read land on 8 different units, and the two rows of one
-//    parity that a transposed read touches (x differing in its lowest bit) on different
-//    halves of the row.
+// no LDS stores; layout in lds_rows.hpp), two stages deep: the next listed tile moves while
+// the current one is consumed, behind one wait and one barrier per tile.
 // LDS of both kernels: two stages of two tiles, then per stage 1 KB of row vectors (at 0 and
 // 256: two vectors of 64 floats; at 512: the partial tile's bitmap, or without bitmaps the
 // original numbers of the tile's rows, and in stage 0 at 768 the mask's terms).
 template <int D>
-struct Tile {
-  static constexpr int ROW = 2 * D;             // bytes of a row
-  static constexpr int UPR = D / 8;             // 16-byte units of a row
-  static constexpr int RPI = 64 / UPR;          // rows a DMA instruction moves
-  static constexpr int NI = 16 / RPI;           // instructions per tensor and wave (16 rows)
-  static constexpr int TB = kBT * ROW;          // bytes of a staged tile
+struct Tile : Rows<D> {
+  static constexpr int TB = kBT * Rows<D>::ROW;          // bytes of a staged tile
   static constexpr int STAGE = 2 * TB;
   static constexpr int VEC = 1024;
   static constexpr int VEC_OFF = 2 * STAGE;
   static constexpr int TERMS_OFF = VEC_OFF + 768;
   static constexpr int END = VEC_OFF + 2 * VEC;
   static_assert(PA_MAX_TERMS * sizeof(pa_term) <= 256, "the terms fit beside the row numbers");
-  __device__ static int swz(int r) {
-    return D == 128 ? 4 * (r & 3) + ((r >> 2) & 3) : 4 * ((r >> 1) & 1) + ((r >> 2) & 3);
-  }
 };
 
-typedef const __attribute__((address_space(3))) f32x4 lds_f4;
-typedef __attribute__((address_space(3))) f32x4 lds_f4w;
-typedef __attribute__((address_space(3))) u32x4 lds_u4w;
 typedef const __attribute__((address_space(3))) int32_t lds_i32;
 typedef __attribute__((address_space(3))) float lds_fw;
-typedef const __attribute__((address_space(4))) int32_t cint;
 typedef const __attribute__((address_space(4))) int8_t cbyte;
-
-// Per-lane LDS geometry of the reads of 32 staged rows (offsets of stage, tile and chunk are
-// immediates on top of these).  With 256-byte rows, units 8 apart and blocks 2 apart differ
-// in address bit 7 alone, so the upper half of the addresses is the lower half with that
-// bit flipped: one VALU operation at the read instead of eight registers held through
-// the loop.
-template <int D>
-struct TileReads {
-  static constexpr int NR = D == 128 ? 4 : D / 16, NT = 2;
-  lds_cptr row_[NR];     // 16-byte row reads: row m, unit 2 kc + G
-  lds_cptr tr_[NT][2];   // transposed reads of block db: rows 4 G + j16 / 4 (+8)
-  // (volatile, or the flips would be hoisted out of the loop into registers again)
-  __device__ __forceinline__ static lds_cptr flip(lds_cptr p) {
-    uint32_t x;
-    asm volatile("v_xor_b32 %0, 0x80, %1" : "=v"(x) : "v"((uint32_t)(uintptr_t)p));
-    return (lds_cptr)(uintptr_t)x;
-  }
-  __device__ __forceinline__ lds_cptr row(int kc) const { return kc < NR ? row_[kc] : flip(row_[kc - NR]); }
-  __device__ __forceinline__ lds_cptr tr(int db, int s) const { return db < NT ? tr_[db][s] : flip(tr_[db - NT][s]); }
-};
-
-template <int D>
-__device__ __forceinline__ TileReads<D> tile_reads(lds_cptr lds, int lane) {
-  TileReads<D> t;
-  const int m = lane & 31, G = lane >> 5, j16 = lane & 15, h16 = (lane >> 4) & 1;
-#pragma unroll
-  for (int kc = 0; kc < TileReads<D>::NR; ++kc) {
-    t.row_[kc] = lds + m * Tile<D>::ROW + 16 * ((2 * kc + G) ^ Tile<D>::swz(m));
-    // (opaque, so each address stays whole in one register)
-    asm volatile("" : "+v"(t.row_[kc]));
-  }
-#pragma unroll
-  for (int db = 0; db < TileReads<D>::NT; ++db)
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int R = 4 * G + (j16 >> 2) + 8 * s;
-      const int u = 4 * db + 2 * h16 + ((j16 & 3) >> 1);
-      t.tr_[db][s] = lds + R * Tile<D>::ROW + 16 * (u ^ Tile<D>::swz(R)) + 8 * (j16 & 1);
-      asm volatile("" : "+v"(t.tr_[db][s]));
-    }
-  return t;
-}
-
-// A operand X^T of 16 rows of a staged tile at byte offset `off` (stage + tile + first row):
-// the transposed product's fragment for block db of D.
-template <typename T, int D>
-__device__ __forceinline__ typename Mma<T>::frag tr_frag(const TileReads<D>& t, int db, int off) {
-  const s16x4 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t.tr(db, 0) + off));
-  const s16x4 x2 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t.tr(db, 1) + off));
-  const uint4 vx = {__builtin_bit_cast(uint2, x1).x, __builtin_bit_cast(uint2, x1).y, __builtin_bit_cast(uint2, x2).x,
-                    __builtin_bit_cast(uint2, x2).y};
-  return __builtin_bit_cast(typename Mma<T>::frag, vx);
-}
 
 // DMA of rows 16 w .. 16 w + 15 of a tile of two tensors (heads applied; the tile's first
 // row at byte r0b, its rows `pitch` bytes apart: the row pitch, or s times it when the tile
-// is gathered through the residue-s basis) into the stage at LDS m0.  Instruction i writes
-// rows 16 w + RPI i + l / UPR, lane l unit l % UPR, fetching the unit the swizzle stores
-// there (dvoff[i]).
-template <int D>
-__device__ __forceinline__ void dma_offsets(uint32_t* dvoff, int64_t pitch, int lane) {
-  const int r = lane / Tile<D>::UPR, u = lane % Tile<D>::UPR;
-#pragma unroll
-  for (int i = 0; i < Tile<D>::NI; ++i)
-    dvoff[i] = (uint32_t)(r * pitch) + 16u * (uint32_t)(u ^ Tile<D>::swz(Tile<D>::RPI * i + r));
-}
+// is gathered through the residue-s basis) into the stage at LDS m0 (dvoff: dma_offsets).
 template <int D>
 __device__ __forceinline__ void dma_tiles(uint32_t m0, const char* g0, const char* g1, int64_t pitch, int64_t r0b, int w,
                                           const uint32_t* dvoff) {
@@ -313,15 +231,6 @@ __device__ __forceinline__ void store_rows(const BwdK& a, char* smem, const f32x
     if (a.accumulate) x += __builtin_convertvector(__builtin_bit_cast(typename O::t8, old.x[j]), f32x8);
     *O::at(a, head, row0, tid, j) = __builtin_convertvector(x, typename O::t8);
   }
-}
-
-// Issue position -> list position of a launch's n lists, longest first: every second run of
-// 32 goes backwards.  Work-groups are placed round-robin over an XCD's 32 CUs, so a CU whose
-// first list is among the longest of its run then takes the shortest of the next one.
-__device__ __forceinline__ int snake(int p, int n) {
-  const int r0 = p & ~31;
-  const int len = n - r0 < 32 ? n - r0 : 32;
-  return (p & 32) ? r0 + len - 1 - (p & 31) : p;
 }
 
 // ---------------------------------------------------------------------------------

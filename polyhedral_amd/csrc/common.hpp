@@ -145,4 +145,14 @@ __device__ __forceinline__ uint32_t xcd_remap32(uint32_t hw, uint32_t total) {
   return x * per + x + per;
 }
 
+
+// Issue position -> list position of a launch's n lists, longest first: every second run of
+// 32 goes backwards.  Work-groups are placed round-robin over an XCD's 32 CUs, so a CU whose
+// first list is among the longest of its run then takes the shortest of the next one.
+__device__ __forceinline__ int snake(int p, int n) {
+  const int r0 = p & ~31;
+  const int len = n - r0 < 32 ? n - r0 : 32;
+  return (p & 32) ? r0 + len - 1 - (p & 31) : p;
+}
+
 }  // namespace pa

@@ -1,0 +1,109 @@
+"""The f16 / bf16 kernel on plain block lists (pa_attn_fwd_tile, BQ = 64 and 128) against the
+general kernel on the same arguments, over tile shapes, bases, bitmaps, strides and both sides
+of the rule that gives a list two groups of waves.  The two agree up to the rounding of P to 16 bits: it happens at the running maximum,
+which differs between them, so an output element moves by at most 2 eps sum p |v| <= 2 eps
+max |v|, and by an ulp of its own rounding."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import permute as op
+from polyhedral_amd import attention as pattn
+from polyhedral_amd import index as pindex
+from polyhedral_amd.polyattn import masks as pm
+from polyhedral_amd.registry import numpy_mask, triton_params
+from tests.util import make_qkv
+
+pytestmark = pytest.mark.gpu
+
+EPS = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _both(q, k, v, lists, kind, BQ, A, **kw):
+    BH, N, _ = q.shape
+    out = []
+    for general in (False, True):
+        lse = torch.full((BH, N), 7.0, device=q.device)
+        launch = pattn.prepare(q, k, v, *lists, *kind, BQ, A, kernel="general", lse=lse, **kw)
+        assert launch.entry == "pa_attn_fwd"
+        if not general:
+            launch.entry = "pa_attn_fwd_tile"
+        with torch.cuda.device(q.device):
+            o = launch()
+        out.append((o.float(), lse))
+    (o1, l1), (o2, l2) = out
+    eps = EPS[q.dtype]
+    bound = 2 * eps * float(v.float().abs().max()) + 2 * eps * o2.abs()
+    assert bool(((o1 - o2).abs() <= bound).all()), f"output differs by {float((o1 - o2).abs().max()):.2e}"
+    assert torch.equal(torch.isneginf(l1), torch.isneginf(l2))
+    fin = ~torch.isneginf(l2)
+    assert float((l1[fin] - l2[fin]).abs().max()) < 2e-5 if bool(fin.any()) else True
+
+
+def _built(mask, N, BQ, A, gpu):
+    """(lists, wave codes, bitmaps) of a mask."""
+    kv_idx, kv_num, kv_partial, wave, _, _, bits = pindex.build_device(mask, N, BQ, A, device=gpu, bits=True)
+    return (kv_idx, kv_num, kv_partial), wave, bits
+
+
+@pytest.mark.parametrize("bitmaps", [True, False])
+@pytest.mark.parametrize("BQ,A", [(128, 16), (128, 32), (128, 128), (64, 16), (64, 64), (64, 128)])
+@pytest.mark.parametrize("name,D,dtype,BH,N", [
+    ("causal", 64, torch.float16, 3, 1152),            # odd list lengths, two groups of waves
+    ("local256+str8", 64, torch.bfloat16, 2, 640),
+    ("sinks4+win256", 128, torch.bfloat16, 2, 1152),
+    ("twoband-1000", 128, torch.float16, 2, 2176),     # 34 segments apart: lists past 16 steps with gaps
+    ("causal", 64, torch.bfloat16, 130, 1024),         # 1040 / 2080 work-groups: one group
+    ("window-128", 128, torch.float16, 40, 1152),      # 360 / 720
+])
+def test_equals_general_kernel(gpu, name, D, dtype, BH, N, BQ, A, bitmaps):
+    q, k, v = (x.to(gpu) for x in make_qkv(BH, N, D, dtype, seed=N + A))
+    lists, wave, bits = _built(numpy_mask(name), N, BQ, A, gpu)
+    _both(q, k, v, lists, triton_params(name), BQ, A, kv_wave_bits=wave, kv_bits=bits if bitmaps else None,
+          heads_desc=bitmaps)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("BQ,A", [(128, 32), (64, 64)])
+def test_bases_strides_order_and_merge(gpu, BQ, A, D):
+    """A table permutation of the mask alone, the closed-form residue basis gathered and
+    scattered, rows that are not adjacent in memory, an issue order, and a merge input."""
+    BH, N, s, name = 3, 2048, 8, "dilated-8"
+    g = torch.Generator().manual_seed(D)
+    # [N, BH, D] storage: row stride BH * D
+    q, k, v = (torch.randn(N, BH, D, generator=g).to(torch.float16).to(gpu).transpose(0, 1) for _ in range(3))
+    p = op.residue_perm(N, s)
+    perm = torch.from_numpy(p).to(gpu)
+    lists, wave, bits = _built(pm.Permuted(numpy_mask(name), p), N, BQ, A, gpu)
+    order = torch.from_numpy(np.random.default_rng(1).permutation(N // BQ).astype(np.int32)).to(gpu)
+    kind = triton_params(name)
+    for kb in (bits, None):
+        _both(q, k, v, lists, kind, BQ, A, kv_wave_bits=wave, kv_bits=kb, perm_q=perm, qblock_order=order)
+        prev = (torch.randn(BH, N, D, generator=torch.Generator().manual_seed(3)).to(torch.float16).to(gpu),
+                torch.randn(BH, N, generator=torch.Generator().manual_seed(4)).to(gpu))
+        _both(q, k, v, lists, kind, BQ, A, kv_wave_bits=wave, kv_bits=kb, perm_q=perm, gather_q=True, gather_kv=True,
+              scatter_o=True, residue=s, prev=prev)
+    # no wave codes: the partial flags alone
+    _both(q, k, v, lists, kind, BQ, A, kv_bits=bits, perm_q=perm)
+
+
+@pytest.mark.parametrize("BQ", [64, 128])
+def test_dead_rows_and_empty_lists(gpu, BQ):
+    from polyhedral_amd.spec import device_mask
+    N, D = 1024, 64
+    M = numpy_mask("window-128").dense(N).copy()
+    M[5] = False
+    M[256:384] = False
+    q, k, v = (x.to(gpu) for x in make_qkv(2, N, D, torch.float16, seed=1))
+    dm = device_mask(pm.DenseMask(M), N, gpu)
+    lists, wave, bits = _built(pm.DenseMask(M), N, BQ, 64, gpu)
+    for kb in (bits, None):
+        lse = torch.empty(2, N, device=gpu)
+        launch = pattn.prepare(q, k, v, *lists, dm, 0, 0, 0, BQ, 64, kv_wave_bits=wave, kv_bits=kb, lse=lse)
+        assert launch.entry == "pa_attn_fwd_tile"
+        with torch.cuda.device(gpu):
+            o = launch()
+        dead = torch.zeros(N, dtype=torch.bool, device=gpu)
+        dead[5] = dead[256:384] = True
+        assert torch.count_nonzero(o[:, dead]) == 0 and torch.isneginf(lse[:, dead]).all()
+        assert torch.isfinite(o).all() and torch.isfinite(lse[:, ~dead]).all()
