@@ -260,9 +260,8 @@ typedef struct pa_attn_args {
 
 int pa_attn_fwd(const pa_attn_args* args, void* stream);
 
-/* pa_attn_fwd_tile: the same attention by the kernel for f16 / bf16 block lists as they are
- * (no step descriptors; kv_wave_bits and the bitmaps optional), BQ = 64 or 128, any A, D = 64
- * or 128, with any gather_q / scatter_o / prev_o / order, and gather_kv through the
+/* pa_attn_fwd_tile: the same attention by the kernels for f16 / bf16 block lists as they are
+ * (no step descriptors; kv_wave_bits and the bitmaps optional), any tile, with any gather_q / scatter_o / prev_o / order, and gather_kv through the
  * closed-form residue basis only; gather_mult <= 1, no kv_steps, run_groups or wave_split.
  * Results within the rounding of P to 16 bits of pa_attn_fwd's without kv_steps. */
 int pa_attn_fwd_tile(const pa_attn_args* args, void* stream);

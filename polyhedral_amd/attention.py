@@ -31,9 +31,8 @@ streaming kernel whenever its preconditions hold and the index carries its array
 "stream": require it; "general": the general kernel).
 
 The HIP kernels that serve the call: the streaming kernel (f16 / bf16, D = 128, BQ = 128,
-A in 16, 32, 64) moves K and V into LDS by DMA and masks from bitmaps; the tile kernel
-(f16 / bf16, BQ = 64 or 128, "auto" only) does so from the plain lists, with or without
-bitmaps; the wave-split kernel takes small float32 grids; the general kernel takes every
+A in 16, 32, 64) moves K and V into LDS by DMA and masks from bitmaps; the tile kernels
+(f16 / bf16, "auto" only) do so from the plain lists, with or without bitmaps; the wave-split kernel takes small float32 grids; the general kernel takes every
 other shape and dtype and can evaluate the predicate itself.
 """
 import ctypes
@@ -297,10 +296,11 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
         args.wsel, args.wsel_sb = _lib.ptr(wsel_t), wsel_t.stride(0)
     keep = [q, k, v, o, kv_idx, kv_num, kv_partial, kv_wave_bits, kv_bits, dmask, lse, prev, qblock_order,
             kv_steps, wsel_t, run]
-    # the tile kernel (pa_attn_fwd_tile) takes the 2-byte types' plain lists; measured against
-    # the general kernel over its range it is 1.4 to 3 times as fast (attn_tile.hip)
+    # the tile kernels (pa_attn_fwd_tile) take the 2-byte types' plain lists; measured against
+    # the general kernel over their range they are 1.4 to 5 times as fast (attn_tile.hip,
+    # attn_narrow.hip)
     use_tile = (kernel == "auto" and not (use_stream or use_ws) and q.dtype in (torch.float16, torch.bfloat16) and
-                BQ in (64, 128) and gather_mult == 1 and not (gathers_kv and not residue))
+                gather_mult == 1 and not (gathers_kv and not residue))
     return Launch(args, keep, o, dev,
                   "run" if use_run else "stream" if use_stream else "wsplit" if use_ws else "general",
                   "pa_attn_fwd_tile" if use_tile else "pa_attn_fwd")

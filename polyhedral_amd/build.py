@@ -21,7 +21,8 @@ LIB = LIBDIR / "libpolyattn_amd.so"
 ARCH = "gfx950"
 
 SOURCES = ["common.hip", "index.hip", "permute.hip", "merge.hip", "attn_fwd.hip",
-           "attn_bf16.hip", "attn_f16.hip", "attn_f32.hip", "attn_stream.hip", "attn_wsplit.hip", "attn_tile.hip", "decode.hip", "bwd.hip"]
+           "attn_bf16.hip", "attn_f16.hip", "attn_f32.hip", "attn_stream.hip", "attn_wsplit.hip", "attn_tile.hip", "attn_narrow.hip",
+           "decode.hip", "bwd.hip"]
 
 # -packed-fp32-ops: keep the compiler from emitting v_pk_{add,mul,fma}_f32.
 HIP_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-mcode-object-version=5",
@@ -44,10 +45,11 @@ def _torch_lib():
     return pathlib.Path(spec.origin).parent / "lib"
 
 
-# per-source additions: the streaming and tile kernels compute no NaN on purpose (masked scores
+# per-source additions: the streaming, tile and narrow kernels compute no NaN on purpose (masked scores
 # are -inf, never NaN), so fmax needs no NaN-quieting instructions
 EXTRA_FLAGS = {"attn_stream.hip": ["-fno-honor-nans", "-Wno-inline-asm"],
-               "attn_tile.hip": ["-fno-honor-nans", "-Wno-inline-asm"], "bwd.hip": ["-Wno-inline-asm"], "decode.hip": ["-Wno-inline-asm"]}
+               "attn_tile.hip": ["-fno-honor-nans", "-Wno-inline-asm"],
+               "attn_narrow.hip": ["-fno-honor-nans", "-Wno-inline-asm"], "bwd.hip": ["-Wno-inline-asm"], "decode.hip": ["-Wno-inline-asm"]}
 
 
 def _compile(src, hipcc):

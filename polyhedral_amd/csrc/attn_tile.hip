@@ -5,8 +5,8 @@
 // _attn_fwd, gpu/triton_attn.py:62-182): scores transposed (S^T = K Q^T) on 32x32x16 MFMAs,
 // online softmax with the finite -1e30 sentinel and a lazy rescale, probabilities rounded
 // to 16 bits only as MFMA operands (their sum is taken in fp32 before), the l > 0 guard, and
-// the log-sum-exp merge with a previous partial.  attn_fwd_kernel stages K and V through
-// registers and keeps the rest: f32, BQ <= 32, K / V gathered through a permutation table,
+// the log-sum-exp merge with a previous partial (narrower query blocks: attn_narrow.hip).  attn_fwd_kernel stages K and V through
+// registers and keeps the rest: f32, K / V gathered through a permutation table,
 // class-B emulation.
 //
 // A work-group is RG row groups (BQ / 32, one wave of 32 query rows each) times KG key
@@ -492,12 +492,15 @@ int launch_tile_d(const AttnK& a, hipStream_t s) {
 
 }  // namespace
 
+// 2-byte types, rows gathered in index space or through the closed-form basis
 bool attn_tile_takes(const AttnK& a, int dtype) {
-  return (dtype == PA_F16 || dtype == PA_BF16) && (a.BQ == 64 || a.BQ == 128) && a.gather_mult <= 1 &&
-         !(a.gather_kv && a.residue_s == 0);
+  return (dtype == PA_F16 || dtype == PA_BF16) && a.gather_mult <= 1 && !(a.gather_kv && a.residue_s == 0);
 }
 
+int launch_attn_narrow(const AttnK& a, int dtype, int D, hipStream_t s);
+
 int launch_attn_tile(const AttnK& a, int dtype, int D, hipStream_t s) {
+  if (a.BQ < 64) return launch_attn_narrow(a, dtype, D, s);
   if (dtype == PA_BF16) return D == 64 ? launch_tile_d<__bf16, 64>(a, s) : launch_tile_d<__bf16, 128>(a, s);
   return D == 64 ? launch_tile_d<_Float16, 64>(a, s) : launch_tile_d<_Float16, 128>(a, s);
 }

@@ -1,4 +1,4 @@
-"""The f16 / bf16 kernel on plain block lists (pa_attn_fwd_tile, BQ = 64 and 128) against the
+"""The f16 / bf16 kernels on plain block lists (pa_attn_fwd_tile) against the
 general kernel on the same arguments, over tile shapes, bases, bitmaps, strides and both sides
 of the rule that gives a list two groups of waves.  The two agree up to the rounding of P to 16 bits: it happens at the running maximum,
 which differs between them, so an output element moves by at most 2 eps sum p |v| <= 2 eps
@@ -47,7 +47,8 @@ def _built(mask, N, BQ, A, gpu):
 
 
 @pytest.mark.parametrize("bitmaps", [True, False])
-@pytest.mark.parametrize("BQ,A", [(128, 16), (128, 32), (128, 128), (64, 16), (64, 64), (64, 128)])
+@pytest.mark.parametrize("BQ,A", [(128, 16), (128, 32), (128, 128), (64, 16), (64, 64), (64, 128),
+                                  (32, 16), (32, 32), (32, 128), (16, 16), (16, 32), (16, 64)])
 @pytest.mark.parametrize("name,D,dtype,BH,N", [
     ("causal", 64, torch.float16, 3, 1152),            # odd list lengths, two groups of waves
     ("local256+str8", 64, torch.bfloat16, 2, 640),
@@ -64,7 +65,7 @@ def test_equals_general_kernel(gpu, name, D, dtype, BH, N, BQ, A, bitmaps):
 
 
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("BQ,A", [(128, 32), (64, 64)])
+@pytest.mark.parametrize("BQ,A", [(128, 32), (64, 64), (32, 32), (16, 16)])
 def test_bases_strides_order_and_merge(gpu, BQ, A, D):
     """A table permutation of the mask alone, the closed-form residue basis gathered and
     scattered, rows that are not adjacent in memory, an issue order, and a merge input."""
@@ -87,7 +88,7 @@ def test_bases_strides_order_and_merge(gpu, BQ, A, D):
     _both(q, k, v, lists, kind, BQ, A, kv_bits=bits, perm_q=perm)
 
 
-@pytest.mark.parametrize("BQ", [64, 128])
+@pytest.mark.parametrize("BQ", [16, 32, 64, 128])
 def test_dead_rows_and_empty_lists(gpu, BQ):
     from polyhedral_amd.spec import device_mask
     N, D = 1024, 64
@@ -107,3 +108,13 @@ def test_dead_rows_and_empty_lists(gpu, BQ):
         dead[5] = dead[256:384] = True
         assert torch.count_nonzero(o[:, dead]) == 0 and torch.isneginf(lse[:, dead]).all()
         assert torch.isfinite(o).all() and torch.isfinite(lse[:, ~dead]).all()
+
+
+@pytest.mark.parametrize("N", [16, 48, 80])
+def test_narrow_blocks_of_a_short_sequence(gpu, N):
+    """Heads whose 16-row units do not fill a work-group of four."""
+    for D in (64, 128):
+        q, k, v = (x.to(gpu) for x in make_qkv(3, N, D, torch.bfloat16, seed=N))
+        lists, wave, bits = _built(numpy_mask("causal"), N, 16, 16, gpu)
+        for kb in (bits, None):
+            _both(q, k, v, lists, triton_params("causal"), 16, 16, kv_wave_bits=wave, kv_bits=kb)
