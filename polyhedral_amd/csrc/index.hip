@@ -3,10 +3,17 @@
 // mask on the host and tiles it with numpy any/all.
 //
 // Phase 1 (classify): work-groups (query block, column split) walk the KV columns in
-// chunks of 256 (split j takes chunks j, j + splits, ...), evaluate the predicate for
-// the block's BQ rows and fold the result into per-tile codes: 2 bits (some live / all
-// live) per wave group of 32 query rows x min(A, 32) columns.  Wave ballots do the
-// column reduction; a query block's list length is summed over its splits.
+// chunks of 256 (split j takes chunks j, j + splits, ...) and fold the predicate over
+// the block's BQ rows into per-tile codes: 2 bits (some live / all live) per wave group
+// of 32 query rows x min(A, 32) columns.  Most blocks of 32 rows x a wave's 64 columns are
+// live or dead as a whole, which the ranges of their original positions (and, for strided
+// terms, their common residues) decide, and most chunks of columns in order so too; the
+// rest are evaluated pair by pair (an explicit matrix: every pair).  Wave ballots
+// do the column reduction; a query block's list length is summed over its splits.
+// Evaluating every pair was bound by the VALU: the classification of a prefix-LM at N =
+// 16256, 128x32 tiles, took 304 us against 50, at 65536 4810 against 130, lattice-16 outside
+// a band in its basis at 16384 533 against 114; what remains is the mixed blocks and, in a
+// table basis, the ranges.
 // Phase 2 (compact): one work-group per query block scans the tile codes and
 // writes the ascending, zero-padded kv_idx / kv_partial / kv_wave_bits rows.
 #include "common.hpp"
@@ -23,12 +30,115 @@ __global__ void zero_totals_kernel(unsigned long long* totals, int32_t* kv_num, 
   if (i < nq) kv_num[i] = 0;
 }
 
-// The longest list, once every split has added its count.
+// The listed tiles and the longest list, once every split has added its count.
 __global__ void max_list_kernel(const int32_t* kv_num, int32_t nq, unsigned long long* totals) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   int32_t v = i < nq ? kv_num[i] : 0;
-  for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_down(v, off, 64));
-  if ((threadIdx.x & 63) == 0 && v > 0) atomicMax(&totals[2], (unsigned long long)v);
+  unsigned long long sum = (unsigned long long)v;
+  for (int off = 32; off > 0; off >>= 1) {
+    v = max(v, __shfl_down(v, off, 64));
+    sum += __shfl_down(sum, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0 && v > 0) {
+    atomicAdd(&totals[0], sum);
+    atomicMax(&totals[2], (unsigned long long)v);
+  }
+}
+
+// What a set of pairs is under a term or the whole predicate: kMixed = not decided here.
+enum Verdict { kDead, kLive, kMixed };
+
+// A block of rows and columns in original positions: their ranges, and for a stride p
+// whether each side has one residue (rq, rk).
+struct Range {
+  int32_t q0, q1, k0, k1;
+};
+
+// Decides a term for every pair of the block at once where its ranges allow; `same(p)` is 1
+// when all rows and all columns have one residue mod p, 0 when each side has one and they
+// differ, -1 otherwise.
+template <typename F>
+__device__ __forceinline__ Verdict term_verdict(const pa_term& t, const Range& r, F same) {
+  const int64_t d0 = (int64_t)r.q0 - r.k1, d1 = (int64_t)r.q1 - r.k0;  // range of q - kv
+  auto strided = [&](int32_t p) -> Verdict {                           // d % p == 0, given d >= 0
+    const int s = same(p);
+    return s == 1 ? kLive : s == 0 ? kDead : kMixed;
+  };
+  switch (t.kind) {
+    case PA_FULL:
+      return kLive;
+    case PA_PREFIX_LM:
+      if (d0 >= 0 || (r.q1 < t.p0 && r.k1 < t.p0)) return kLive;
+      return (d1 < 0 && (r.q0 >= t.p0 || r.k0 >= t.p0)) ? kDead : kMixed;
+    case PA_DENSE:
+      return kMixed;
+    default:
+      break;
+  }
+  // the other kinds are causal
+  if (d1 < 0) return kDead;
+  if (t.kind == PA_DILATED) {
+    const Verdict v = strided(t.p0);
+    return (v == kLive && d0 < 0) ? kMixed : v;
+  }
+  if (d0 < 0) {
+    // pairs on both sides of the diagonal: dead only where no d >= 0 of the range is live
+    return kMixed;
+  }
+  switch (t.kind) {
+    case PA_CAUSAL:
+      return kLive;
+    case PA_WINDOW:
+      return d1 < t.p0 ? kLive : d0 >= t.p0 ? kDead : kMixed;
+    case PA_LOCAL_STRIDED:
+      if (d1 < t.p0) return kLive;
+      {
+        const Verdict v = strided(t.p1);
+        return v == kLive ? kLive : d0 >= t.p0 ? v : kMixed;
+      }
+    case PA_TWOBAND: {
+      // (the band's end wraps as term_live's 32-bit sum does)
+      const int64_t b0 = t.p1, b1 = (int32_t)((uint32_t)t.p1 + (uint32_t)t.p2);
+      if (d1 < t.p0 || (d0 >= b0 && d1 < b1)) return kLive;
+      return (d0 >= t.p0 && (d0 >= b1 || d1 < b0)) ? kDead : kMixed;
+    }
+    case PA_SINKS:
+      if (d1 < t.p0 || r.k1 < t.p1) return kLive;
+      return (d0 >= t.p0 && r.k0 >= t.p1) ? kDead : kMixed;
+    default:
+      return kMixed;
+  }
+}
+
+// The whole predicate: live where an include term is and no exclude term is.
+template <typename F>
+__device__ __forceinline__ Verdict pred_verdict(const Pred& p, const Range& r, F same) {
+  Verdict inc = kDead, exc = kDead;
+  const int n = p.n_include + p.n_exclude;
+#pragma unroll
+  for (int i = 0; i < PA_MAX_TERMS; ++i) {  // (constant indices into the argument block)
+    if (i < n) {
+      const Verdict v = term_verdict(p.terms[i], r, same);
+      Verdict& to = i < p.n_include ? inc : exc;
+      if (v == kLive || to == kLive)
+        to = kLive;
+      else if (v == kMixed)
+        to = kMixed;
+    }
+  }
+  if (inc == kDead || exc == kLive) return kDead;
+  return (inc == kLive && exc == kDead) ? kLive : kMixed;
+}
+
+__device__ __forceinline__ int32_t wave_min(int32_t x) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) x = min(x, __shfl_xor(x, o));
+  return x;
+}
+__device__ __forceinline__ int32_t wave_max_i(int32_t x) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) x = max(x, __shfl_xor(x, o));
+  return x;
 }
 
 __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int32_t N, int32_t BQ,
@@ -39,6 +149,7 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int
   __shared__ uint32_t tile_code[kChunk / 16];
   __shared__ int32_t red_live[kThreads / 64];
   __shared__ int32_t red_tiles;
+  __shared__ int32_t q_lo[4], q_hi[4];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -57,26 +168,89 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int
   }
   if (tid == 0) red_tiles = 0;
   __syncthreads();
+  if (wave < n_rg) {
+    // the row groups' ranges (their rows, one per lane; lanes past them repeat)
+    const int32_t qo = q_orig[wave * rg_rows + (lane & (rg_rows - 1))];
+    const int32_t lo = wave_min(qo), hi = wave_max_i(qo);
+    if (lane == 0) {
+      q_lo[wave] = lo;
+      q_hi[wave] = hi;
+    }
+  }
+  __syncthreads();
 
   int32_t live_count = 0;
   int32_t tiles_listed = 0;  // meaningful in thread 0 only
+  // pairs and tiles of the chunks decided at once (thread 0's count)
+  long long live_whole = 0;
+  int32_t tiles_whole = 0;
+  const int log2a = 31 - __builtin_clz((unsigned)A), log2cw = 31 - __builtin_clz((unsigned)cw);
+  Range rw;
+  rw.q0 = q_lo[0];
+  rw.q1 = q_hi[0];
+  for (int g = 1; g < n_rg; ++g) {
+    rw.q0 = min(rw.q0, q_lo[g]);
+    rw.q1 = max(rw.q1, q_hi[g]);
+  }
+  const uint32_t all_code = n_rg * ncg == 16 ? ~0u : (1u << (2 * n_rg * ncg)) - 1u;
 
   for (int c0 = split * kChunk; c0 < N; c0 += splits * kChunk) {
+    if (!pred.perm_kv) {
+      // a chunk of columns in order that is live or dead as a whole (uniform: no barrier)
+      rw.k0 = c0;
+      rw.k1 = min(c0 + kChunk, N) - 1;
+      const Verdict v = pred_verdict(pred, rw, [](int32_t p) -> int { return p == 1 ? 1 : -1; });
+      if (v != kMixed) {
+        const int cols = rw.k1 - c0 + 1, tiles = cols >> log2a;
+        if (tid < tiles) codes[(int64_t)qb * nk + (c0 >> log2a) + tid] = v == kLive ? all_code : 0u;
+        if (v == kLive) {
+          live_whole += (long long)cols * BQ;
+          tiles_whole += tiles;
+        }
+        continue;
+      }
+    }
     if (tid < kChunk / 16) tile_code[tid] = 0u;
     __syncthreads();
 
     const int col = c0 + tid;
     const bool valid = col < N;
     uint32_t any_rg = 0u, all_rg = 0u;
-    if (valid) {
-      const int32_t ko = pred.perm_kv ? pred.perm_kv[col] : col;
+    if (c0 + wave * 64 < N) {  // (uniform; lane 0's column is then valid)
+      int32_t ko = valid ? (pred.perm_kv ? pred.perm_kv[col] : col) : 0;
+      const int32_t ko0 = __shfl(ko, 0);
+      if (!valid) ko = ko0;  // a lane past the end stands for a column of the block
+      Range r;
+      if (pred.perm_kv) {
+        r.k0 = wave_min(ko);
+        r.k1 = wave_max_i(ko);
+      } else {
+        r.k0 = c0 + wave * 64;
+        r.k1 = min(c0 + wave * 64 + 64, N) - 1;
+      }
       for (int g = 0; g < n_rg; ++g) {
-        bool any = false, all = true;
-        for (int rr = 0; rr < rg_rows; ++rr) {
-          const bool live = pred_live(pred, q_orig[g * rg_rows + rr], ko);
-          any |= live;
-          all &= live;
-          live_count += live ? 1 : 0;
+        const int32_t qo = q_orig[g * rg_rows + (lane & (rg_rows - 1))];
+        r.q0 = q_lo[g];
+        r.q1 = q_hi[g];
+        const Verdict v = pred_verdict(pred, r, [&](int32_t p) -> int {
+          const int32_t rq = qo % p, rk = ko % p;
+          const int32_t rq0 = __builtin_amdgcn_readfirstlane(rq), rk0 = __builtin_amdgcn_readfirstlane(rk);
+          if (__ballot(rq != rq0 || rk != rk0) != 0ull) return -1;
+          return rq0 == rk0 ? 1 : 0;
+        });
+        bool any = v == kLive, all = v == kLive;
+        if (v == kMixed) {
+          all = true;
+          int32_t n = 0;
+          for (int rr = 0; rr < rg_rows; ++rr) {
+            const bool live = pred_live(pred, q_orig[g * rg_rows + rr], ko);
+            any |= live;
+            all &= live;
+            n += live ? 1 : 0;
+          }
+          if (valid) live_count += n;
+        } else if (v == kLive && valid) {
+          live_count += rg_rows;
         }
         any_rg |= (any ? 1u : 0u) << g;
         all_rg |= (all ? 1u : 0u) << g;
@@ -94,17 +268,17 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int
           const unsigned long long gm = (cw == 64 ? ~0ull : ((1ull << cw) - 1ull)) << (lane * cw);
           const bool gany = (b_any & gm) != 0ull;
           const bool gall = (b_all & gm) == gm;
-          const int cg = (gc0 % A) / cw;
+          const int cg = (gc0 & (A - 1)) >> log2cw;
           const int code_g = g * ncg + cg;
           const uint32_t bits = (gany ? 1u : 0u) << (2 * code_g) | (gall ? 1u : 0u) << (2 * code_g + 1);
-          if (bits) atomicOr(&tile_code[(gc0 - c0) / A], bits);
+          if (bits) atomicOr(&tile_code[(gc0 - c0) >> log2a], bits);
         }
       }
     }
     __syncthreads();
-    const int tiles_in_chunk = kChunk / A;
+    const int tiles_in_chunk = kChunk >> log2a;
     if (tid < tiles_in_chunk) {
-      const int kb = c0 / A + tid;
+      const int kb = (c0 >> log2a) + tid;
       if (kb < nk) {
         const uint32_t code = tile_code[tid];
         codes[(int64_t)qb * nk + kb] = code;
@@ -119,13 +293,10 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int
   if (lane == 0) red_live[wave] = live_count;
   __syncthreads();
   if (tid == 0) {
-    long long tot = 0;
+    long long tot = live_whole;
     for (int i = 0; i < kThreads / 64; ++i) tot += red_live[i];
-    tiles_listed = red_tiles;
-    if (tiles_listed) {
-      atomicAdd(&kv_num[qb], tiles_listed);
-      atomicAdd(&totals[0], (unsigned long long)tiles_listed);
-    }
+    tiles_listed = red_tiles + tiles_whole;
+    if (tiles_listed) atomicAdd(&kv_num[qb], tiles_listed);
     if (tot) atomicAdd(&totals[1], (unsigned long long)tot);
   }
 }
@@ -198,7 +369,8 @@ extern "C" int pa_index_classify(const pa_mask* mask, int64_t N, int32_t BQ, int
   hipLaunchKernelGGL(pa::zero_totals_kernel, dim3((unsigned)((nq + 3 + 255) / 256)), dim3(256), 0, s, totals, kv_num,
                      (int32_t)nq);
   PA_LAUNCH_CHECK("zero_totals_kernel");
-  // enough column splits for about 2048 work-groups (the chip holds ~2048 of 256 threads)
+  // enough column splits for about 2048 work-groups (the chip holds ~2048 of 256 threads;
+  // 1024 were 10 to 45% slower)
   const int64_t chunks = (N + pa::kChunk - 1) / pa::kChunk;
   int64_t splits = (2048 + nq - 1) / nq;
   if (splits > chunks) splits = chunks;
@@ -235,9 +407,11 @@ extern "C" int pa_index_compact(const uint32_t* tile_codes, const int32_t* kv_nu
 }
 
 // ---------------------------------------------------------------------------
-// Element bitmaps of the listed partial tiles (phase 3).  One work-group per query
-// block walks its list; each partial tile gets BQ x ceil(A/32) words, one thread per
-// word, 32 predicate evaluations per word.
+// Element bitmaps of the listed partial tiles (phase 3).  One work-group per query block
+// takes its list 256 entries at a time, one per thread: the flags are ranked with ballots
+// (one dependent load per 256 entries, not per entry) and the partial tiles collected in
+// LDS; then each gets BQ x ceil(A/32) words, one thread per word, 32 predicate evaluations
+// per word.
 namespace pa {
 namespace {
 
@@ -258,18 +432,30 @@ __global__ __launch_bounds__(kThreads) void bits_kernel(const Pred pred, int32_t
     q_orig[tid] = pred.perm_q ? pred.perm_q[r] : r;
   }
   __syncthreads();
+  __shared__ int32_t part_kb[kThreads];
+  __shared__ int32_t wave_tot[kThreads / 64];
+  const int lane = tid & 63, wave = tid >> 6;
   const int n = kv_num[qb];
   const int64_t row = (int64_t)qb * pitch;
   int64_t rank = part_base[qb];
-  for (int j = 0; j < n; ++j) {
-    const bool partial = kv_partial[row + j] != 0;
-    if (tid == 0) kv_bits_off[row + j] = partial ? (int32_t)(rank * words) : -1;
-    if (!partial) continue;
-    const int kb = kv_idx[row + j];
-    uint32_t* dst = pool + rank * words;
-    for (int wi = tid; wi < words; wi += kThreads) {
+  for (int j0 = 0; j0 < n; j0 += kThreads) {
+    const int j = j0 + tid;
+    const bool partial = j < n && kv_partial[row + j] != 0;
+    const unsigned long long bal = __ballot(partial);
+    if (lane == 0) wave_tot[wave] = __popcll(bal);
+    __syncthreads();
+    int before = __popcll(bal & ((1ull << lane) - 1ull)), total = 0;
+    for (int i = 0; i < kThreads / 64; ++i) {
+      if (i < wave) before += wave_tot[i];
+      total += wave_tot[i];
+    }
+    if (j < n) kv_bits_off[row + j] = partial ? (int32_t)((rank + before) * words) : -1;
+    if (partial) part_kb[before] = kv_idx[row + j];
+    __syncthreads();
+    for (int x = tid; x < total * words; x += kThreads) {
+      const int u = x / words, wi = x - u * words;
       const int rr = wi / wpr, cw = wi % wpr;
-      const int c0 = kb * A + cw * 32;
+      const int c0 = part_kb[u] * A + cw * 32;
       const int ncol = A - cw * 32 < 32 ? A - cw * 32 : 32;
       uint32_t bits = 0u;
       for (int c = 0; c < ncol; ++c) {
@@ -277,9 +463,10 @@ __global__ __launch_bounds__(kThreads) void bits_kernel(const Pred pred, int32_t
         const int32_t ko = pred.perm_kv ? pred.perm_kv[col] : col;
         bits |= (pred_live(pred, q_orig[rr], ko) ? 1u : 0u) << c;
       }
-      dst[wi] = bits;
+      pool[(rank + u) * words + wi] = bits;
     }
-    ++rank;
+    __syncthreads();  // part_kb and wave_tot are read
+    rank += total;
   }
   for (int64_t j = n + tid; j < pitch; j += kThreads) kv_bits_off[row + j] = -1;
 }
