@@ -90,6 +90,12 @@ int pa_index_classify(const pa_mask* mask, int64_t N, int32_t BQ, int32_t A,
                       uint32_t* tile_codes /* [N/BQ * N/A] */, int32_t* kv_num /* [N/BQ] */,
                       unsigned long long* totals /* [3] */, void* stream);
 
+/* Partial tiles of the query blocks before each one: part_base[i] = listed tiles of blocks
+ * 0 .. i - 1 that are not full (from the codes), i = 0 .. N/BQ; part_base[N/BQ] is their
+ * total.  Lets a caller size pa_index_bits' pool together with the lists (one read-back of
+ * totals and part_base). */
+int pa_index_part_base(const uint32_t* tile_codes, int64_t N, int32_t BQ, int32_t A, int64_t* part_base, void* stream);
+
 /* Compacts the codes into ascending kv tile lists, zero padded to `pitch` columns:
  * kv_idx int32 [N/BQ, pitch], kv_partial int8 [N/BQ, pitch] (1 = not full),
  * kv_wave_bits uint32 [N/BQ, pitch] (the tile code; may be NULL). */

@@ -79,6 +79,7 @@ SIGNATURES = {
     "pa_last_error": (ctypes.c_char_p, []),
     "pa_abi_version": (c_i32, []),
     "pa_index_classify": (ctypes.c_int, [ctypes.POINTER(PaMask), c_i64, c_i32, c_i32, c_vp, c_vp, c_vp, c_vp]),
+    "pa_index_part_base": (ctypes.c_int, [c_vp, c_i64, c_i32, c_i32, c_vp, c_vp]),
     "pa_index_compact": (ctypes.c_int, [c_vp, c_vp, c_i64, c_i32, c_i32, c_vp, c_vp, c_vp, c_i64, c_vp]),
     "pa_index_bits": (ctypes.c_int, [ctypes.POINTER(PaMask), c_i64, c_i32, c_i32, c_vp, c_vp, c_vp, c_i64, c_vp,
                                      c_vp, c_vp, c_vp]),
@@ -143,13 +144,19 @@ def check(rc, what):
 def require_device(*tensors):
     """Every tensor must live on a HIP device: the kernels have no host path."""
     for t in tensors:
-        if t is not None and (not isinstance(t, torch.Tensor) or t.device.type != "cuda"):
+        if t is not None and (not isinstance(t, torch.Tensor) or not t.is_cuda):
             dev = t.device if isinstance(t, torch.Tensor) else type(t).__name__
             raise RuntimeError(f"polyhedral_amd kernels run on the GPU only; got a tensor on {dev}")
 
 
 def stream_of(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    # (the current stream's handle without a Stream object)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(t.device.index))
+
+
+def address(t):
+    """A tensor's address for a pointer field (None: NULL), without a ctypes object."""
+    return t.data_ptr() if t is not None else None
 
 
 def ptr(t):

@@ -58,6 +58,16 @@ def _assert_kinds_match():
         raise RuntimeError(f"kind constants diverged: triton_attn={mine} masks_gpu={theirs}")
 
 
+_KINDS_CHECKED = False
+
+
+def _check_kinds_once():
+    """The constants of both modules are fixed once imported: compared at the first call."""
+    global _KINDS_CHECKED
+    _assert_kinds_match()
+    _KINDS_CHECKED = True
+
+
 def _rows3(t, name):
     if t.dim() != 3:
         raise ValueError(f"{name} must be [BH, N, D]")
@@ -99,6 +109,8 @@ def block_sparse_attention(q, k, v, kv_idx, kv_num, kv_partial,
     evaluate the mask in original coordinates (identity when None)."""
     launch = prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale, perm_q, perm_kv,
                      gather_kv, gather_mult, gather_scatter, num_warps, num_stages, **ext)
+    if launch.device.index == torch.cuda.current_device():
+        return launch()
     with torch.cuda.device(launch.device):
         return launch()
 
@@ -118,7 +130,8 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
     BH, N, D = q.shape
     if perm_kv is None:
         perm_kv = perm_q
-    _assert_kinds_match()
+    if not _KINDS_CHECKED:
+        _check_kinds_once()
     assert N % BQ == 0 and N % A == 0, "cost model and kernel both assume this"
     assert k.shape == v.shape == q.shape
     if int(gather_mult) < 1:
@@ -141,7 +154,9 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
     if kv_wave_bits is None:
         kv_wave_bits = wave_bits_for(kv_idx, BQ, A)
     if kv_wave_bits is not None:
-        kv_wave_bits = kv_wave_bits.to(torch.int32).contiguous()
+        if kv_wave_bits.dtype != torch.int32:
+            kv_wave_bits = kv_wave_bits.to(torch.int32)
+        kv_wave_bits = kv_wave_bits.contiguous()
         if kv_wave_bits.shape != kv_idx.shape:
             raise ValueError("kv_wave_bits must have the shape of kv_idx")
     if kernel not in ("auto", "stream", "general", "wsplit"):
@@ -178,28 +193,30 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
     if o.shape != q.shape or o.dtype != q.dtype:
         raise ValueError("out must match q in shape and dtype")
 
+    ptr = _lib.address
     args = _lib.PaAttnArgs()
-    args.q, args.k, args.v, args.o = _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o)
-    args.q_sb, args.q_sn = q.stride(0), q.stride(1)
-    args.k_sb, args.k_sn = k.stride(0), k.stride(1)
-    args.v_sb, args.v_sn = v.stride(0), v.stride(1)
-    args.o_sb, args.o_sn = o.stride(0), o.stride(1)
+    args.q, args.k, args.v, args.o = q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr()
+    args.q_sb, args.q_sn, _ = q.stride()
+    args.k_sb, args.k_sn, _ = k.stride()
+    args.v_sb, args.v_sn, _ = v.stride()
+    args.o_sb, args.o_sn, _ = o.stride()
     args.BH, args.N, args.D = BH, N, D
     args.dtype = _lib.dtype_code(q)
     args.scale = float(scale or D ** -0.5)
     args.BQ, args.A = BQ, A
-    args.kv_idx, args.kv_num, args.kv_partial = _lib.ptr(kv_idx), _lib.ptr(kv_num), _lib.ptr(kv_partial)
-    args.kv_wave_bits = _lib.ptr(kv_wave_bits)
+    args.kv_idx, args.kv_num, args.kv_partial = ptr(kv_idx), ptr(kv_num), ptr(kv_partial)
+    args.kv_wave_bits = ptr(kv_wave_bits)
     args.pitch = kv_idx.shape[1]
     if kv_bits is not None:
         bits_off, bits_pool = kv_bits
         _lib.require_device(bits_off, bits_pool)
         if bits_off.shape != kv_idx.shape or bits_off.dtype != torch.int32 or bits_pool.dtype != torch.int32:
             raise ValueError("kv_bits must be (int32 offsets shaped like kv_idx, int32 bitmap pool)")
-        args.kv_bits_off, args.kv_bits = _lib.ptr(bits_off), _lib.ptr(bits_pool)
+        args.kv_bits_off, args.kv_bits = ptr(bits_off), ptr(bits_pool)
     args.mask = dmask.struct()
     gathers_kv = bool(gather_kv) and (perm_kv is not None or bool(residue))
-    args.gather_q, args.gather_kv, args.scatter_o = int(bool(gather_q)), int(gathers_kv), int(bool(scatter_o))
+    if gather_q or gathers_kv or scatter_o:
+        args.gather_q, args.gather_kv, args.scatter_o = int(bool(gather_q)), int(gathers_kv), int(bool(scatter_o))
     if residue:
         # perm_q = perm_kv = residue_perm(N, residue), evaluated in closed form by the kernel
         qn = N // residue
@@ -210,7 +227,7 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
         _lib.require_device(lse)
         if lse.dtype != torch.float32 or lse.shape != (BH, N) or lse.stride(1) != 1:
             raise ValueError("lse must be float32 [BH, N] with unit row stride")
-        args.lse, args.lse_sb = _lib.ptr(lse), lse.stride(0)
+        args.lse, args.lse_sb = ptr(lse), lse.stride(0)
     if prev is not None:
         o_prev, lse_prev = prev
         _lib.require_device(o_prev, lse_prev)
@@ -221,15 +238,15 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
             raise ValueError("lse and prev lse must share their row stride")
         if lse_prev.stride(1) != 1:
             raise ValueError("prev lse needs a unit row stride")
-        args.prev_o, args.prev_dtype = _lib.ptr(o_prev), _lib.dtype_code(o_prev)
+        args.prev_o, args.prev_dtype = ptr(o_prev), _lib.dtype_code(o_prev)
         args.prev_sb, args.prev_sn = o_prev.stride(0), o_prev.stride(1)
-        args.prev_lse = _lib.ptr(lse_prev)
+        args.prev_lse = ptr(lse_prev)
         args.lse_sb = lse_prev.stride(0)
     if qblock_order is not None:
         qblock_order = qblock_order.to(device=dev, dtype=torch.int32).contiguous()
         if qblock_order.numel() != nq:
             raise ValueError("qblock_order must have N/BQ entries")
-        args.qblock_order = _lib.ptr(qblock_order)
+        args.qblock_order = ptr(qblock_order)
     # the streaming kernel's preconditions (pa_attn_fwd rejects kv_steps otherwise)
     pitch = kv_idx.shape[1]
     why = None
@@ -251,7 +268,7 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
         if kv_steps.dtype != torch.int32 or kv_steps.dim() != 3 or kv_steps.shape[0] != nq \
                 or kv_steps.shape[2] != 16 or not kv_steps.is_contiguous():
             raise ValueError("kv_steps must be contiguous int32 [N/BQ, steps, 16]")
-        args.kv_steps, args.steps_pitch = _lib.ptr(kv_steps), kv_steps.shape[1]
+        args.kv_steps, args.steps_pitch = ptr(kv_steps), kv_steps.shape[1]
     use_run = use_stream and run is not None
     if use_run:
         # run = (schedule, the piece of its rows this call is)
@@ -262,7 +279,7 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
         for t, n in ((k, "k"), (v, "v")):
             if t.stride(0) != N * t.stride(1):
                 raise ValueError(f"the persistent kernel needs {n} with batch stride N * row stride")
-        args.run_steps, args.run_start, args.run_groups = _lib.ptr(run.run), _lib.ptr(run.start), run.groups
+        args.run_steps, args.run_start, args.run_groups = ptr(run.run), ptr(run.start), run.groups
     # the wave-split kernel (pa_attn_args.wave_split): float32 grids of fewer query blocks
     # than the chip has CUs, where one work-group per block would leave most of it idle
     why_ws = None
@@ -279,8 +296,10 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
         raise ValueError(f"the wave-split kernel cannot take this call: {why_ws}")
     use_ws = (not use_stream and why_ws is None and
               (kernel == "wsplit" or (kernel == "auto" and BH * nq < WSPLIT_MAX_BLOCKS)))
-    args.wave_split = 1 if use_ws else 0
-    args.heads_desc = 1 if heads_desc else 0
+    if use_ws:
+        args.wave_split = 1
+    if heads_desc:
+        args.heads_desc = 1
     wsel_t = None
     if gather_mult > 1:
         # [1, 0, ...] per batch-head, as gpu/triton_attn.py:202-205: runtime weights keep the
@@ -293,7 +312,7 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
             if wsel_t.shape != (BH, gather_mult):
                 raise ValueError(f"wsel must be [BH, gather_mult] = [{BH}, {gather_mult}]")
         args.gather_mult, args.gather_scatter = gather_mult, 1 if gather_scatter else 0
-        args.wsel, args.wsel_sb = _lib.ptr(wsel_t), wsel_t.stride(0)
+        args.wsel, args.wsel_sb = ptr(wsel_t), wsel_t.stride(0)
     keep = [q, k, v, o, kv_idx, kv_num, kv_partial, kv_wave_bits, kv_bits, dmask, lse, prev, qblock_order,
             kv_steps, wsel_t, run]
     # the tile kernels (pa_attn_fwd_tile) take the 2-byte types' plain lists; measured against

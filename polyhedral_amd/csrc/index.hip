@@ -348,6 +348,60 @@ __global__ __launch_bounds__(kThreads) void compact_kernel(const uint32_t* __res
   }
 }
 
+// Partial tiles of each query block, then their exclusive prefix sum.
+__global__ __launch_bounds__(kThreads) void part_count_kernel(const uint32_t* __restrict__ codes, int32_t nk,
+                                                               uint32_t full_mask, int64_t* __restrict__ part_base) {
+  __shared__ int32_t tot[kThreads / 64];
+  const int tid = threadIdx.x;
+  const uint32_t* row = codes + (int64_t)blockIdx.x * nk;
+  int32_t n = 0;
+  for (int k = tid; k < nk; k += kThreads) {
+    const uint32_t c = row[k];
+    n += ((c & 0x55555555u) != 0u && (c & full_mask) != full_mask) ? 1 : 0;
+  }
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
+  if ((tid & 63) == 0) tot[tid >> 6] = n;
+  __syncthreads();
+  if (tid == 0) {
+    for (int i = 1; i < kThreads / 64; ++i) n += tot[i];
+    part_base[blockIdx.x] = n;
+  }
+}
+
+__global__ __launch_bounds__(kThreads) void part_scan_kernel(int64_t* part_base, int32_t nq) {
+  __shared__ long long wave_tot[kThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  long long base = 0;
+  for (int i0 = 0; i0 < nq; i0 += kThreads) {
+    const int i = i0 + tid;
+    const long long n = i < nq ? (long long)part_base[i] : 0;
+    long long sum = n;  // inclusive within the wave
+    for (int off = 1; off < 64; off <<= 1) {
+      const long long y = __shfl_up(sum, off, 64);
+      if (lane >= off) sum += y;
+    }
+    if (lane == 63) wave_tot[wave] = sum;
+    __syncthreads();
+    long long before = base, total = 0;
+    for (int u = 0; u < kThreads / 64; ++u) {
+      if (u < wave) before += wave_tot[u];
+      total += wave_tot[u];
+    }
+    if (i < nq) part_base[i] = before + sum - n;
+    base += total;
+    __syncthreads();
+  }
+  if (tid == 0) part_base[nq] = base;
+}
+
+// The codes' all-live bits of a tile.
+uint32_t full_mask_of(int32_t BQ, int32_t A) {
+  const int ngroups = (BQ / (BQ < 32 ? BQ : 32)) * (A / (A < 32 ? A : 32));
+  uint32_t m = 0u;
+  for (int g = 0; g < ngroups; ++g) m |= 2u << (2 * g);
+  return m;
+}
+
 bool tile_ok(int32_t x) { return x == 16 || x == 32 || x == 64 || x == 128; }
 
 }  // namespace
@@ -384,6 +438,22 @@ extern "C" int pa_index_classify(const pa_mask* mask, int64_t N, int32_t BQ, int
   return PA_OK;
 }
 
+extern "C" int pa_index_part_base(const uint32_t* tile_codes, int64_t N, int32_t BQ, int32_t A, int64_t* part_base,
+                                  void* stream) {
+  PA_CHECK_ARG(tile_codes && part_base, "pa_index_part_base: null argument");
+  PA_CHECK_ARG(N >= 1 && N <= (1ll << 30), "pa_index_part_base: N=%lld out of range", (long long)N);
+  PA_CHECK_ARG(pa::tile_ok(BQ) && pa::tile_ok(A) && N % BQ == 0 && N % A == 0,
+               "pa_index_part_base: bad tile shape BQ=%d A=%d for N=%lld", BQ, A, (long long)N);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int32_t nq = (int32_t)(N / BQ);
+  hipLaunchKernelGGL(pa::part_count_kernel, dim3((unsigned)nq), dim3(pa::kThreads), 0, s, tile_codes, (int32_t)(N / A),
+                     pa::full_mask_of(BQ, A), part_base);
+  PA_LAUNCH_CHECK("part_count_kernel");
+  hipLaunchKernelGGL(pa::part_scan_kernel, dim3(1), dim3(pa::kThreads), 0, s, part_base, nq);
+  PA_LAUNCH_CHECK("part_scan_kernel");
+  return PA_OK;
+}
+
 extern "C" int pa_index_compact(const uint32_t* tile_codes, const int32_t* kv_num, int64_t N, int32_t BQ,
                                 int32_t A, int32_t* kv_idx, int8_t* kv_partial, uint32_t* kv_wave_bits,
                                 int64_t pitch, void* stream) {
@@ -394,11 +464,7 @@ extern "C" int pa_index_compact(const uint32_t* tile_codes, const int32_t* kv_nu
   PA_CHECK_ARG(pitch >= 0, "pa_index_compact: negative pitch");
   if (pitch == 0) return PA_OK;  // every query block is empty: nothing to write
   PA_CHECK_ARG(kv_idx && kv_partial, "pa_index_compact: null output");
-  const int rg_rows = BQ < 32 ? BQ : 32;
-  const int cw = A < 32 ? A : 32;
-  const int ngroups = (BQ / rg_rows) * (A / cw);
-  uint32_t full_mask = 0u;
-  for (int g = 0; g < ngroups; ++g) full_mask |= 2u << (2 * g);
+  const uint32_t full_mask = pa::full_mask_of(BQ, A);
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(pa::compact_kernel, dim3((unsigned)(N / BQ)), dim3(pa::kThreads), 0, s, tile_codes,
                      kv_num, (int32_t)N, BQ, A, full_mask, kv_idx, kv_partial, kv_wave_bits, pitch);

@@ -145,24 +145,24 @@ class KVCache:
         if o.shape != q.shape or o.dtype != q.dtype:
             raise ValueError("out must match q in shape and dtype")
         a = _lib.PaDecodeArgs()
-        a.q, a.q_sb, a.q_sn, a.nq, a.qpos0 = _lib.ptr(q), q.stride(0), q.stride(1), nq, qpos0
-        a.k_cache, a.v_cache = _lib.ptr(self.k), _lib.ptr(self.v)
+        a.q, a.q_sb, a.q_sn, a.nq, a.qpos0 = q.data_ptr(), q.stride(0), q.stride(1), nq, qpos0
+        a.k_cache, a.v_cache = self.k.data_ptr(), self.v.data_ptr()
         a.c_sb, a.c_sn = self.k.stride(0), self.k.stride(1)
         a.capacity, a.length, a.residue_s = self.capacity, L, self.residue
         a.mask = dm.struct()
         a.BH, a.D, a.dtype = BH, D, _lib.dtype_code(q)
         a.scale = float(scale) if scale else float(D ** -0.5)
-        a.o, a.o_sb, a.o_sn = _lib.ptr(o), o.stride(0), o.stride(1)
+        a.o, a.o_sb, a.o_sn = o.data_ptr(), o.stride(0), o.stride(1)
         keep_new = []
         if n_new:
-            a.k_new, a.v_new, a.new_sb, a.new_sn = _lib.ptr(k_new), _lib.ptr(v_new), k_new.stride(0), k_new.stride(1)
+            a.k_new, a.v_new, a.new_sb, a.new_sn = k_new.data_ptr(), v_new.data_ptr(), k_new.stride(0), k_new.stride(1)
             a.n_new, a.new_pos0 = n_new, new_pos0
             keep_new = [k_new, v_new]
         if lse is not None:
             _lib.require_device(lse)
             if lse.dtype != torch.float32 or lse.shape != (BH, nq) or lse.stride(1) != 1:
                 raise ValueError("lse must be float32 [BH, nq] with unit stride")
-            a.lse, a.lse_sb = _lib.ptr(lse), lse.stride(0)
+            a.lse, a.lse_sb = lse.data_ptr(), lse.stride(0)
         # the split partials' size is known before any state changes: a static call that
         # would not fit the library's scratch is refused here, not at launch time
         nbytes = ctypes.c_int64(0)
@@ -174,7 +174,7 @@ class KVCache:
             launch = DecodeLaunch(a, [q, o, lse, dm, self.k, self.v] + keep_new, o, dev, static_scratch=True)
         else:
             ws = torch.empty(max(1, (nbytes.value + 3) // 4), dtype=torch.float32, device=dev)
-            a.workspace, a.workspace_bytes = _lib.ptr(ws), ws.numel() * 4
+            a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel() * 4
             launch = DecodeLaunch(a, [q, o, lse, dm, ws, self.k, self.v] + keep_new, o, dev)
         self.length = total
         return launch
@@ -186,6 +186,8 @@ class KVCache:
         before = self.length
         launch = self.prepare(q, mask, scale, qpos0, out, lse, length, static_scratch, k_new, v_new)
         try:
+            if self.device.index == torch.cuda.current_device():
+                return launch()
             with torch.cuda.device(self.device):
                 return launch()
         except Exception:

@@ -135,29 +135,37 @@ def build_device(mask, N, BQ, A, *, perm=None, perm_kv=None, device=None, bits=F
     dm = device_mask(mask, N, dev, perm=perm, perm_kv=perm_kv)
     nq, nk = N // BQ, N // A
     codes = torch.empty(nq * nk, dtype=torch.int32, device=dev)
+    # totals [3] and the partial tiles before each query block [nq + 1], read back together
+    head = torch.empty(4 + nq, dtype=torch.int64, device=dev)
+    totals, part_base = head[:3], head[3:]
     kv_num = torch.empty(nq, dtype=torch.int32, device=dev)
-    totals = torch.empty(3, dtype=torch.int64, device=dev)
     L = _lib.lib()
     ms = dm.struct()
     with torch.cuda.device(dev):
         stream = _lib.stream_of(codes)
         _lib.check(L.pa_index_classify(ctypes.byref(ms), N, BQ, A, _lib.ptr(codes), _lib.ptr(kv_num), _lib.ptr(totals),
                                        stream), "pa_index_classify")
-        tiles, live, max_kv = (int(x) for x in totals.cpu())
-        kv_idx = torch.empty((nq, max_kv), dtype=torch.int32, device=dev)
-        kv_partial = torch.empty((nq, max_kv), dtype=torch.int8, device=dev)
-        wave = torch.empty((nq, max_kv), dtype=torch.int32, device=dev)
+        if bits:
+            _lib.check(L.pa_index_part_base(_lib.ptr(codes), N, BQ, A, _lib.ptr(part_base), stream),
+                       "pa_index_part_base")
+        back = (head if bits else totals).cpu()
+        tiles, live, max_kv = back[:3].tolist()
+        # one allocation for the lists (the flags last, a byte each), so that build() can
+        # read them back in one copy
+        n = nq * max_kv
+        lists = torch.empty(2 * n + (n + 3) // 4, dtype=torch.int32, device=dev)
+        kv_idx, wave = lists[:n].view(nq, max_kv), lists[n:2 * n].view(nq, max_kv)
+        kv_partial = lists[2 * n:].view(torch.int8)[:n].view(nq, max_kv)
         _lib.check(L.pa_index_compact(_lib.ptr(codes), _lib.ptr(kv_num), N, BQ, A, _lib.ptr(kv_idx),
                                       _lib.ptr(kv_partial), _lib.ptr(wave), max_kv, stream),
                    "pa_index_compact")
         out = (kv_idx, kv_num, kv_partial, wave, tiles, live)
         if bits:
-            part = kv_partial.to(torch.int64).sum(1)
-            part_base = torch.cumsum(part, 0) - part
-            n_part = int(part.sum())
+            # (pa_index_bits writes every offset and every word of the partial tiles)
+            n_part = int(back[-1])
             wpr = (A + 31) // 32
-            pool = torch.zeros(max(1, n_part * BQ * wpr), dtype=torch.int32, device=dev)
-            off = torch.full((nq, max_kv), -1, dtype=torch.int32, device=dev)
+            pool = torch.empty(max(1, n_part * BQ * wpr), dtype=torch.int32, device=dev)
+            off = torch.empty((nq, max_kv), dtype=torch.int32, device=dev)
             _lib.check(L.pa_index_bits(ctypes.byref(ms), N, BQ, A, _lib.ptr(kv_idx), _lib.ptr(kv_num),
                                        _lib.ptr(kv_partial), max_kv, _lib.ptr(part_base), _lib.ptr(off),
                                        _lib.ptr(pool), stream), "pa_index_bits")
@@ -176,8 +184,12 @@ def build(mask, N, BQ, A, *, perm=None, perm_kv=None, device=None):
     stream = (BQ, A) in STREAM_TILES
     kv_idx, kv_num, kv_partial, wave, tiles, live = build_device(mask, N, BQ, A, perm=perm, perm_kv=perm_kv,
                                                                  device=device, steps=stream)[:6]
-    return BlockIndex(BQ, A, N, kv_idx.cpu().numpy(), kv_num.cpu().numpy(), kv_partial.cpu().numpy(),
-                      tiles * BQ * A, live, wave.cpu().numpy().view(np.uint32),
+    # the three lists share one allocation: one copy, then views of it
+    n, shape = kv_idx.numel(), tuple(kv_idx.shape)
+    lists = torch.empty(0, dtype=torch.int32, device=kv_idx.device).set_(kv_idx.untyped_storage()).cpu().numpy()
+    return BlockIndex(BQ, A, N, lists[:n].reshape(shape), kv_num.cpu().numpy(),
+                      lists[2 * n:].view(np.int8)[:n].reshape(shape), tiles * BQ * A, live,
+                      lists[n:2 * n].reshape(shape).view(np.uint32),
                       _device=(kv_idx, kv_num, kv_partial, wave))
 
 

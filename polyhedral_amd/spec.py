@@ -8,6 +8,7 @@ Anything else is materialised through its ``row_cols`` (the reference's own
 method, gpu/blockindex.py:35) into a DENSE bitmap that the GPU then tiles.
 """
 from dataclasses import dataclass, field
+from functools import lru_cache
 
 import numpy as np
 import torch
@@ -36,7 +37,7 @@ class MaskSpec:
         """A spec from the reference's (kind, p0, p1, p2) tuple, or a MaskSpec as-is."""
         if isinstance(kind, MaskSpec):
             return kind
-        return cls(((int(kind), int(p0), int(p1), int(p2)),))
+        return _single(int(kind), int(p0), int(p1), int(p2))
 
     def live(self, q, kv):
         """numpy evaluation of the same predicate (host checks and the flex-style mask)."""
@@ -66,6 +67,21 @@ class MaskSpec:
         for t in self.exclude:
             inc = inc & ~term(t)
         return inc
+
+
+@lru_cache(maxsize=256)
+def _single(kind, p0, p1, p2):
+    return MaskSpec(((kind, p0, p1, p2),))
+
+
+@lru_cache(maxsize=256)
+def _term_struct(include, exclude):
+    """A pa_mask of these terms, without tables (copied by DeviceMask.struct)."""
+    m = _lib.PaMask()
+    m.n_include, m.n_exclude = len(include), len(exclude)
+    for i, t in enumerate(include + exclude):
+        m.terms[i] = _lib.PaTerm(*[int(x) for x in t])
+    return m
 
 
 def _terms_by_name(mask):
@@ -106,14 +122,12 @@ class DeviceMask:
     _keep: list = field(default_factory=list)
 
     def struct(self):
-        m = _lib.PaMask()
-        m.n_include, m.n_exclude = len(self.spec.include), len(self.spec.exclude)
-        for i, t in enumerate(self.spec.include + self.spec.exclude):
-            m.terms[i] = _lib.PaTerm(*[int(x) for x in t])
-        m.perm_q = _lib.ptr(self.perm_q)
-        m.perm_kv = _lib.ptr(self.perm_kv)
-        m.dense_bits = _lib.ptr(self.dense_bits)
-        m.dense_words = int(self.dense_bits.shape[1]) if self.dense_bits is not None else 0
+        m = _lib.PaMask.from_buffer_copy(_term_struct(tuple(map(tuple, self.spec.include)),
+                                                      tuple(map(tuple, self.spec.exclude))))
+        m.perm_q = _lib.address(self.perm_q)
+        m.perm_kv = _lib.address(self.perm_kv)
+        if self.dense_bits is not None:
+            m.dense_bits, m.dense_words = self.dense_bits.data_ptr(), int(self.dense_bits.shape[1])
         return m
 
 
