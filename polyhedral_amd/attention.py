@@ -319,7 +319,8 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
     # the general kernel over their range they are 1.4 to 5 times as fast (attn_tile.hip,
     # attn_narrow.hip)
     use_tile = (kernel == "auto" and not (use_stream or use_ws) and q.dtype in (torch.float16, torch.bfloat16) and
-                gather_mult == 1 and not (gathers_kv and not residue))
+                gather_mult == 1 and not (gathers_kv and not residue) and
+                min(k.stride(1), v.stride(1)) >= 0 and 2 * N * max(k.stride(1), v.stride(1)) < 2 ** 32)
     return Launch(args, keep, o, dev,
                   "run" if use_run else "stream" if use_stream else "wsplit" if use_ws else "general",
                   "pa_attn_fwd_tile" if use_tile else "pa_attn_fwd")

@@ -204,7 +204,8 @@ extern "C" int pa_attn_fwd_tile(const pa_attn_args* x, void* stream) {
   PA_CHECK_ARG(x->run_groups == 0 && !x->wave_split && !x->kv_steps,
                "pa_attn_fwd_tile: takes no run_groups, wave_split or kv_steps");
   PA_CHECK_ARG(pa::attn_tile_takes(a, x->dtype),
-               "pa_attn_fwd_tile: needs f16 or bf16, no K / V gather through a table and no class-B emulation (dtype %d)",
+               "pa_attn_fwd_tile: needs f16 or bf16, no K / V gather through a table, no class-B emulation and a head's K "
+               "and V within 4 GiB (dtype %d)",
                x->dtype);
   return pa::launch_attn_tile(a, x->dtype, x->D, static_cast<hipStream_t>(stream));
 }

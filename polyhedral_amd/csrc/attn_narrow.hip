@@ -23,7 +23,7 @@
 // MFMAs; four waves per SIMD (118 registers) at D = 64 and two (186) at D = 128.  Against
 // attn_fwd_kernel, f16: lattice-8 in its basis, 8 heads x 8192, 16x16 tiles, D = 64 211 ->
 // 45 us (191 live TFLOP/s); window 256, 8 x 8192: 16x16 140 -> 29 us, D = 128 286 -> 54;
-// 32x32 89 -> 31, D = 128 171 -> 58; causal, 8 x 2048: 16x16 128 -> 49, D = 128 241 -> 79;
+// 32x32 89 -> 31, D = 128 171 -> 58; causal, 8 x 2048: 16x16 128 -> 42, D = 128 241 -> 79;
 // 32x32, D = 128 157 -> 81.
 #include <type_traits>
 
@@ -141,7 +141,11 @@ void attn_narrow_kernel(const AttnK a, int units, int groups) {
   // 32 steps of the list: lane l holds segment 64 c + l (its first column, its bitmap
   // offset); bit l of live / full: it has a live pair / is all live.  The next 32 steps'
   // entries are loaded (raw) halfway through these.
+  // (row offsets inside a head are 32-bit, checked on the host: they go into the lanes'
+  // addresses, and the 64-bit bases stay as they are; 64-bit products and sums per step on
+  // the scalar unit took 48.5 us of causal 16x16, 8 x 2048, against 41.9)
   int32_t c_col = 0, c_boff = -1, r_tile = 0, r_boff = -1;
+  uint32_t c_koff = 0u, c_voff = 0u;
   uint32_t r_code = 0u;
   uint64_t c_live = 0ull, c_full = 0ull;
   auto load_raw = [&](int c) __attribute__((always_inline)) {
@@ -166,6 +170,9 @@ void attn_narrow_kernel(const AttnK a, int units, int groups) {
     // (a segment past the list holds its step's other one again, with code 0)
     const int first = __shfl(c_col, lane & ~1);
     if (!in) c_col = first;
+    const int row = gather_kv ? orig_closed(c_col) : c_col;
+    c_koff = (uint32_t)row * (uint32_t)krow_b;
+    c_voff = (uint32_t)row * (uint32_t)vrow_b;
     c_boff = r_boff >= 0 ? r_boff + ((within * 16) >> 5) : -1;
   };
 
@@ -185,20 +192,19 @@ void attn_narrow_kernel(const AttnK a, int units, int groups) {
     s.full = (uint32_t)(c_full >> l0) & 3u;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      s.col[t] = __builtin_amdgcn_readlane(c_col, l0 + t);
-      const int64_t row = gather_kv ? orig_closed(s.col[t]) : s.col[t];
-      const char* kp = kbase + row * krow_b;
+      if (!use_bits) s.col[t] = __builtin_amdgcn_readlane(c_col, l0 + t);
+      const uint32_t ko = koff + (uint32_t)__builtin_amdgcn_readlane((int)c_koff, l0 + t);
+      const uint32_t vo = (uint32_t)__builtin_amdgcn_readlane((int)c_voff, l0 + t);
 #pragma unroll
-      for (int kc = 0; kc < NK; ++kc) d.k[t][kc] = *reinterpret_cast<const u32x4*>(kp + (koff + 64u * kc));
+      for (int kc = 0; kc < NK; ++kc) d.k[t][kc] = *reinterpret_cast<const u32x4*>(kbase + ko + 64 * kc);
       if (use_bits && s.full != 3u) {
         const int bo = __builtin_amdgcn_readlane(c_boff, l0 + t);
         d.word[t] = ((s.full >> t) & 1u)                ? ~0u
-                    : (((s.live >> t) & 1u) && bo >= 0) ? a.kv_bits[(int64_t)bo + row_b * wpr] >> (s.col[t] & 16 & (A - 1))
+                    : (((s.live >> t) & 1u) && bo >= 0) ? a.kv_bits[(int64_t)bo + row_b * wpr] >> (A >= 32 ? 16 * t : 0)
                                                         : 0u;
       }
-      const char* vp = vbase + row * vrow_b;
 #pragma unroll
-      for (int i = 0; i < R::NI; ++i) dma_x4(ring0 + S * STAGE + t * SEG + i * 1024, vp, voff[i]);
+      for (int i = 0; i < R::NI; ++i) dma_x4(ring0 + S * STAGE + t * SEG + i * 1024, vbase, voff[i] + vo);
     }
   };
   // bits 4 g + 0..3 of a partial segment by evaluating the predicate (index without bitmaps)

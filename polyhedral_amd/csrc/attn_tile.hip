@@ -119,14 +119,23 @@ void attn_tile_kernel(const AttnK a) {
   uint32_t koff[R::NI], voff[R::NI];
   dma_offsets<D>(koff, rstride * krow_b, lane);
   dma_offsets<D>(voff, rstride * vrow_b, lane);
-  const int64_t kstep = (int64_t)R::RPI * rstride * krow_b, vstep = (int64_t)R::RPI * rstride * vrow_b;
+  const uint32_t kstep = (uint32_t)(R::RPI * rstride * krow_b), vstep = (uint32_t)(R::RPI * rstride * vrow_b);
+#pragma unroll
+  for (int i = 1; i < R::NI; ++i) {
+    koff[i] += i * kstep;
+    voff[i] += i * vstep;
+  }
 
   // The list, 16 of this key group's steps at a time: lane 4 u + t holds segment t (16
   // columns) of step 16 c + u, its first column, its row in memory and its bitmap offset; the
   // segments' codes for this wave are two 64-bit words (bit 4 u + t: some pair live / every
   // pair live).  A step then costs a few scalar operations.  The next 16 steps' entries are
   // loaded (raw) halfway through these.
+  // (row offsets inside a head are 32-bit, checked on the host: they go into the lanes'
+  // addresses, and the 64-bit bases stay as they are: window 1024, 64x64, bf16 D = 128,
+  // 16 x 8192, 179.5 -> 172.5 us)
   int32_t c_col = 0, c_boff = -1;   // current 16 steps
+  uint32_t c_koff = 0u, c_voff = 0u;
   uint64_t c_live = 0ull, c_full = 0ull;
   int32_t r_idx_ = 0, r_boff = -1;  // raw entries of the next 16
   uint32_t r_code = 0u;
@@ -156,6 +165,9 @@ void attn_tile_kernel(const AttnK a) {
     // query block meets anyway)
     const int first = __shfl(c_col, lane & ~3);
     if (!in) c_col = first;
+    const int row = gather_kv ? orig_closed(c_col) : c_col;
+    c_koff = (uint32_t)row * (uint32_t)krow_b;
+    c_voff = (uint32_t)row * (uint32_t)vrow_b;
     c_boff = r_boff >= 0 ? r_boff + ((within * 16) >> 5) : -1;
   };
 
@@ -169,15 +181,13 @@ void attn_tile_kernel(const AttnK a) {
 #pragma unroll
     for (int u = 0; u < SPW; ++u) {
       const int at = SPW * w + u;
-      const int col = __builtin_amdgcn_readlane(c_col, u4 + at);
-      const int64_t row = gather_kv ? orig_closed(col) : col;
+      const uint32_t ko = (uint32_t)__builtin_amdgcn_readlane((int)c_koff, u4 + at);
+      const uint32_t vo = (uint32_t)__builtin_amdgcn_readlane((int)c_voff, u4 + at);
       const uint32_t m0 = ring0 + (uint32_t)(S * STAGE + at * 16 * R::ROW);
-      const char* kp = kbase + row * krow_b;
-      const char* vp = vbase + row * vrow_b;
 #pragma unroll
       for (int i = 0; i < R::NI; ++i) {
-        dma_x4(m0 + i * 1024, kp + i * kstep, koff[i]);
-        dma_x4(m0 + TB + i * 1024, vp + i * vstep, voff[i]);
+        dma_x4(m0 + i * 1024, kbase, koff[i] + ko);
+        dma_x4(m0 + TB + i * 1024, vbase, voff[i] + vo);
       }
     }
   };
@@ -478,8 +488,8 @@ int launch_tile_t(const AttnK& a, hipStream_t s) {
 //   BQ = 128, D = 64:  64 work-groups 44.1 / 31.5, 256 73.2 / 52.0, 384 93.8 / 67.9; 1024
 //     with short lists fill the chip either way;
 //   BQ = 128, D = 128 (one work-group of two groups per CU by its LDS): 256 107 / 77;
-//   BQ = 64, D = 64:  128 40.8 / 27.2, 512 71.8 / 44.4, 2048 (window 1024) 87.1 / 105;
-//   BQ = 64, D = 128: 512 105 / 95, 2048 (window 1024) 180 / 227.
+//   BQ = 64, D = 64:  128 40.8 / 27.2, 512 71.8 / 44.4, 2048 (window 1024) 85 / 105;
+//   BQ = 64, D = 128: 512 105 / 95, 2048 (window 1024) 172 / 227.
 template <typename T, int D>
 int launch_tile_d(const AttnK& a, hipStream_t s) {
   if (a.BQ == 64) {
@@ -492,9 +502,12 @@ int launch_tile_d(const AttnK& a, hipStream_t s) {
 
 }  // namespace
 
-// 2-byte types, rows gathered in index space or through the closed-form basis
+// 2-byte types, rows gathered in index space or through the closed-form basis, a head's K
+// and V within 4 GiB
 bool attn_tile_takes(const AttnK& a, int dtype) {
-  return (dtype == PA_F16 || dtype == PA_BF16) && a.gather_mult <= 1 && !(a.gather_kv && a.residue_s == 0);
+  const int64_t row = 2 * (a.k_sn > a.v_sn ? a.k_sn : a.v_sn);
+  return (dtype == PA_F16 || dtype == PA_BF16) && a.gather_mult <= 1 && !(a.gather_kv && a.residue_s == 0) &&
+         a.k_sn >= 0 && a.v_sn >= 0 && a.N * row < (1ll << 32);
 }
 
 int launch_attn_narrow(const AttnK& a, int dtype, int D, hipStream_t s);
