@@ -9,9 +9,9 @@
 // registers and keeps the rest: f32, K / V gathered through a permutation table,
 // class-B emulation.
 //
-// A work-group is RG row groups (BQ / 32, one wave of 32 query rows each) times KG key
-// groups.  Key group g takes the 64-column steps g, g + KG, ... of the query block's list,
-// its K and V rows by LDS DMA into a two-stage ring of its own (layout in lds_rows.hpp), the
+// A work-group is RG row groups (one wave of 32 query rows each; all of the query block's, or
+// with H = 2 half of them) times KG key groups.  Key group g takes the 64-column steps g,
+// g + KG, ... of the query block's list, its K and V rows by LDS DMA into a two-stage ring of its own (layout in lds_rows.hpp), the
 // next step's while this one is computed, behind one wait and one barrier per step.  The key
 // groups' states (max, sum, O^T) are merged through LDS at the end.
 //
@@ -19,7 +19,7 @@
 // maxima, sums and packing about 850, so the VALU, as far as three waves per SIMD overlap
 // (causal, 32 heads x 8192, f16: 375 us, 730 TFLOP/s, about 1500 clocks per wave's step); on
 // short lists an item's start and end.  Against attn_fwd_kernel: that case 798 us; 8 heads x
-// 4096 causal, 128x128 tiles, f16, D = 64 (no bitmaps) 138 -> 52 us; lattice-8 in its basis,
+// 4096 causal, 128x128 tiles, f16, D = 64 (no bitmaps) 138 -> 44 us; lattice-8 in its basis,
 // 8 heads x 16384, 128x32 tiles 155 -> 64 us; causal, bf16, D = 128, 8 x 4096, 128x128 tiles
 // 209 -> 77 us.  A step's scalar work decides much of it (the scalar unit is shared by the
 // SIMDs): the list read entry by entry, with its codes worked out per step, took 64 us where
@@ -42,7 +42,7 @@ constexpr int tile_smem_bytes() { return KG * 4 * 64 * Rows<D>::ROW; }
 template <int D>
 constexpr int tile_waves() { return D == 64 ? 3 : 2; }
 
-template <typename T, int D, int RG, int KG>
+template <typename T, int D, int RG, int KG, int H>
 __global__ __launch_bounds__(64 * RG * KG) __attribute__((amdgpu_waves_per_eu(tile_waves<D>())))
 void attn_tile_kernel(const AttnK a) {
   using Frag = typename Mma<T>::frag;
@@ -62,16 +62,19 @@ void attn_tile_kernel(const AttnK a) {
   char* ring = smem + kg * 2 * STAGE;
   const uint32_t ring0 = (uint32_t)(uintptr_t)(lds_char_t*)ring;
 
-  const uint32_t lid = xcd_remap32(blockIdx.x, (uint32_t)a.total_wg);
-  const uint32_t bh_l = lid / (uint32_t)a.nq;
+  const uint32_t lid = xcd_remap32(blockIdx.x, gridDim.x);
+  const int np = H * a.nq;  // pieces of a head
+  const uint32_t bh_l = lid / (uint32_t)np;
   const int64_t bh = a.heads_desc ? a.BH - 1 - bh_l : bh_l;
-  const int qb_lin = (int)(lid - bh_l * (uint32_t)a.nq);
+  const int p_lin = (int)(lid - bh_l * (uint32_t)np);
   // (without an order, the last query blocks first: a causal mask's lists grow along the
   // sequence, and the longest should not be the last to start: 456 -> 375 us for 32 heads of
   // 8192 in f16, D = 64.  Up to 1024 work-groups, which mostly start at once, are also dealt
   // to the CUs long with short: 69.5 -> 64.5 us for the lattice-8 mask below; beyond that it
   // costs 3% of L2 reuse.)
-  const int qb = a.qblock_order ? ((cint*)a.qblock_order)[qb_lin] : a.nq - 1 - (a.total_wg <= 1024 ? snake(qb_lin, a.nq) : qb_lin);
+  const int p = a.qblock_order ? p_lin : np - 1 - (gridDim.x <= 1024 ? snake(p_lin, np) : p_lin);
+  const int qb = a.qblock_order ? ((cint*)a.qblock_order)[p / H] : p / H;
+  const int wb = (p % H) * RG + w;  // this wave's row group in the query block
 
   const int A = a.A, spt_log2 = a.spt_log2, spt_mask = (1 << spt_log2) - 1;
   const int ncg = A >= 32 ? (A >> 5) : 1;   // 32-column groups per tile
@@ -90,7 +93,7 @@ void attn_tile_kernel(const AttnK a) {
   };
   const bool has_pq = closed || a.pred.perm_q;
   const bool gather_kv = a.gather_kv && closed;
-  const int r_idx = qb * (32 * RG) + w * 32 + m;  // index-space query row of this lane
+  const int r_idx = qb * (32 * RG * H) + wb * 32 + m;  // index-space query row of this lane
   int q_orig = r_idx;
   if (has_pq) q_orig = closed ? orig_closed(r_idx) : a.pred.perm_q[r_idx];
   const int r_load = (a.gather_q && has_pq) ? q_orig : r_idx;
@@ -157,7 +160,7 @@ void attn_tile_kernel(const AttnK a) {
     const int seg = seg_of(c);
     const int within = seg & spt_mask;
     const bool in = seg < n_seg;
-    const uint32_t code = in ? r_code >> (2 * (w * ncg + (A >= 32 ? within >> 1 : 0))) : 0u;
+    const uint32_t code = in ? r_code >> (2 * (wb * ncg + (A >= 32 ? within >> 1 : 0))) : 0u;
     c_live = __ballot((code & 1u) != 0u);
     c_full = __ballot((code & 2u) != 0u);
     c_col = r_idx_ * A + within * 16;
@@ -195,7 +198,7 @@ void attn_tile_kernel(const AttnK a) {
   // zeros for a dead one, the bitmap's bits for a partial one
   auto words = [&](const Step& s, uint32_t* wd) __attribute__((always_inline)) {
     if (!use_bits || s.full == 15u) return;
-    const uint32_t* rowp = a.kv_bits + (int64_t)(w * 32 + m) * wpr;
+    const uint32_t* rowp = a.kv_bits + (int64_t)(wb * 32 + m) * wpr;
 #pragma unroll
     for (int lb = 0; lb < 2; ++lb) {
       const uint32_t lv = (s.live >> (2 * lb)) & 3u, fl = (s.full >> (2 * lb)) & 3u;
@@ -465,7 +468,7 @@ void attn_tile_kernel(const AttnK a) {
   if (a.lse && G == 0) a.lse[bh * a.lse_sb + srow] = lse_v;
 }
 
-template <typename T, int D, int RG, int KG>
+template <typename T, int D, int RG, int KG, int H>
 int launch_tile_t(const AttnK& a, hipStream_t s) {
   constexpr int smem = tile_smem_bytes<D, KG>();
   static unsigned long long configured = 0ull;  // the dynamic LDS limit is raised once per device
@@ -473,31 +476,57 @@ int launch_tile_t(const AttnK& a, hipStream_t s) {
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
   if (dev >= 64 || !((configured >> dev) & 1ull)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_tile_kernel<T, D, RG, KG>),
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_tile_kernel<T, D, RG, KG, H>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attn_tile_kernel)");
     if (dev < 64) configured |= 1ull << dev;
   }
-  hipLaunchKernelGGL((attn_tile_kernel<T, D, RG, KG>), dim3((unsigned)a.total_wg), dim3(64 * RG * KG), smem, s, a);
+  hipLaunchKernelGGL((attn_tile_kernel<T, D, RG, KG, H>), dim3((unsigned)(H * a.total_wg)), dim3(64 * RG * KG), smem, s, a);
   PA_LAUNCH_CHECK("attn_tile_kernel");
   return PA_OK;
 }
 
-// Two key groups per list where one would leave the chip waiting for its longest lists.
-// One group / two (us; causal unless said):
-//   BQ = 128, D = 64:  64 work-groups 44.1 / 31.5, 256 73.2 / 52.0, 384 93.8 / 67.9; 1024
-//     with short lists fill the chip either way;
-//   BQ = 128, D = 128 (one work-group of two groups per CU by its LDS): 256 107 / 77;
-//   BQ = 64, D = 64:  128 40.8 / 27.2, 512 71.8 / 44.4, 2048 (window 1024) 85 / 105;
-//   BQ = 64, D = 128: 512 105 / 95, 2048 (window 1024) 172 / 227.
+// How many key groups a list is given and into how many pieces of 64 rows a block of 128 is
+// cut: small launches wait for their longest lists.  Measured (us; causal unless said), 128
+// rows by one key group / 128 rows by two / pieces of 64 rows by two / by four:
+//   D = 64, work-groups of 128 rows:
+//     64 (2 x 4096)   - / 50.5 / 41.8 / 33.2      128 (1 x 16384) - / 183 / 153 / 111
+//     128 (window 200, 4 x 4096) - / 10.7 / 9.3 / 9.3     128 (window 1024) - / 18.4 / 15.2 / 13.5
+//     256 (8 x 4096) 73.2 / 51.7 / 43.5 / 53.6    256 (4 x 8192) - / 91.6 / 76.2 / 96.7
+//     256 (32 x 1024) - / 21.1 / 22.1 / 30.2      256 (window 4096, 4 x 8192) - / 49.5 / 50.5 / 57.7
+//     384 (12 x 4096) 93.8 / 63.9 / 60.8 / 74.0   512 (16 x 4096) - / 64.4 / 72.2 / 94.3
+//   so four key groups and pieces up to 128 work-groups, which then fit one to a CU; up to
+//   384 two groups and pieces where the longest list covers most of the sequence (the lists
+//   then mostly differ, and a CU takes a long and a short piece) and is long enough to pay
+//   for staging it twice;
+//   D = 128: 64 (2 x 4096) - / 70.8 / 58.8, 128 (4 x 4096) - / 71.3 / 60.1, 128 (window 200)
+//     - / 39.9 / 32.4, 160 (5 x 4096) - / 72.2 / 71.0, 160 (10 x 2048) - / 42.6 / 47.0, 256
+//     107 / 74.7 / 89.0 (one work-group of two groups per CU by its LDS).
+// Blocks of 64 rows, one key group / two / four:
+//   D = 64:  128 (8 x 1024) - / 18.4 / 16.9, 256 (8 x 2048) - / 26.6 / 22.6, 256 (4 x 4096) - /
+//     42.6 / 33.9, 512 (8 x 4096) 71.8 / 43.4 / 53.6, 2048 (window 1024) 85 / 105 / -;
+//   D = 128: 512 105 / 95, 2048 (window 1024) 172 / 227.
 template <typename T, int D>
 int launch_tile_d(const AttnK& a, hipStream_t s) {
-  if (a.BQ == 64) {
-    if (a.total_wg <= (D == 64 ? 1024 : 512)) return launch_tile_t<T, D, 2, 2>(a, s);
-    return launch_tile_t<T, D, 2, 1>(a, s);
+  if constexpr (D == 64) {
+    if (a.BQ == 64) {
+      if (a.total_wg <= 256) return launch_tile_t<T, D, 2, 4, 1>(a, s);
+      if (a.total_wg <= 1024) return launch_tile_t<T, D, 2, 2, 1>(a, s);
+      return launch_tile_t<T, D, 2, 1, 1>(a, s);
+    }
+    if (a.total_wg <= 128) return launch_tile_t<T, D, 2, 4, 2>(a, s);
+    const int64_t longest = a.pitch * a.A;
+    if (a.total_wg <= 384 && longest >= 2048 && 4 * longest >= 3 * (int64_t)a.N) return launch_tile_t<T, D, 2, 2, 2>(a, s);
+    if (a.total_wg <= 512) return launch_tile_t<T, D, 4, 2, 1>(a, s);
+  } else {
+    if (a.BQ == 64) {
+      if (a.total_wg <= 512) return launch_tile_t<T, D, 2, 2, 1>(a, s);
+      return launch_tile_t<T, D, 2, 1, 1>(a, s);
+    }
+    if (a.total_wg <= 128) return launch_tile_t<T, D, 2, 2, 2>(a, s);
+    if (a.total_wg <= 256) return launch_tile_t<T, D, 4, 2, 1>(a, s);
   }
-  if (a.total_wg <= (D == 64 ? 512 : 256)) return launch_tile_t<T, D, 4, 2>(a, s);
-  return launch_tile_t<T, D, 4, 1>(a, s);
+  return launch_tile_t<T, D, 4, 1, 1>(a, s);
 }
 
 }  // namespace

@@ -1,6 +1,6 @@
 """The f16 / bf16 kernels on plain block lists (pa_attn_fwd_tile) against the
 general kernel on the same arguments, over tile shapes, bases, bitmaps, strides and both sides
-of the rule that gives a list two groups of waves.  The two agree up to the rounding of P to 16 bits: it happens at the running maximum,
+of the rules that give a list groups of waves and cut a block into pieces.  The two agree up to the rounding of P to 16 bits: it happens at the running maximum,
 which differs between them, so an output element moves by at most 2 eps sum p |v| <= 2 eps
 max |v|, and by an ulp of its own rounding."""
 import numpy as np
@@ -56,6 +56,9 @@ def _built(mask, N, BQ, A, gpu):
     ("twoband-1000", 128, torch.float16, 2, 2176),     # 34 segments apart: lists past 16 steps with gaps
     ("causal", 64, torch.bfloat16, 130, 1024),         # 1040 / 2080 work-groups: one group
     ("window-128", 128, torch.float16, 40, 1152),      # 360 / 720
+    ("causal", 64, torch.float16, 9, 2048),            # 144 with long lists: blocks of 128 rows in two pieces
+    ("window-128", 64, torch.bfloat16, 20, 1152),      # 180 / 360 with short ones: whole blocks, two groups
+    ("window-128", 128, torch.bfloat16, 20, 1152),
 ])
 def test_equals_general_kernel(gpu, name, D, dtype, BH, N, BQ, A, bitmaps):
     q, k, v = (x.to(gpu) for x in make_qkv(BH, N, D, dtype, seed=N + A))
