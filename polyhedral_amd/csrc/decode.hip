@@ -28,6 +28,7 @@ namespace {
 
 constexpr int kDecMaxQ = 8;     // query rows per call
 constexpr int kDecWaves = 4;    // waves per work-group
+constexpr int kOneWaves = 8;    // the same of the single-query kernel
 constexpr int kDecTarget = 512;    // work-groups a split plan aims for (two per CU, one round)
 constexpr int kMergeMax = kDecTarget;  // splits per (head, query) the merge takes
 constexpr int kMaxResidue = 4096;       // classes of the largest residue basis a cache may use
@@ -124,14 +125,36 @@ __device__ __forceinline__ float wave_sum(float x) {
   return x;
 }
 
+// The appended rows this work-group owns (entry e of this class's segment in one of its
+// groups) go to the cache: thread u copies 16-byte unit u % NC of the K (u < NC) or V
+// row.  Nothing in this launch reads them back from the cache: the keys' lanes take them
+// from k_new / v_new.
+template <int NC>
+__device__ __forceinline__ void copy_new_rows(const DecK& a, int64_t bh, int split, int tid, int64_t rowb,
+                                              const char* knew, const char* vnew, int esz) {
+  for (int64_t j = 0; j < a.n_new; ++j) {
+    const uint32_t t = (uint32_t)(a.new_pos0 + j);  // (below 2^31, group numbers below 2^32)
+    const uint32_t e = t / (uint32_t)a.s;
+    const uint32_t ncls = t - e * (uint32_t)a.s;
+    if ((ncls * (uint32_t)a.groups + (e >> 8)) % (uint32_t)a.n_split != (uint32_t)split) continue;
+    if (tid < 2 * NC) {
+      const int uu = tid % NC;
+      const char* src = (tid < NC ? knew : vnew) + j * a.new_sn + 16 * uu;
+      char* dst = (tid < NC ? a.k : a.v) + (bh * a.c_sb + ncls * a.Q * a.c_sn) * esz + e * rowb + 16 * uu;
+      *reinterpret_cast<du4*>(dst) = *reinterpret_cast<const du4*>(src);
+    }
+  }
+}
+
 // One work-group per (split, head).  Wave w takes the blocks b0 = 256 k + 64 w of the
 // groups (class, k) the split takes.  LIST: it lists the blocks' live keys, then, 64 listed
 // keys at a time, lane l scores key l from its K row; else lane l scores key b0 + l of each
 // block that holds a live key.  The keys' V rows go by LDS DMA into the wave's 64-row
-// buffer, and for P.V the lanes own output dimensions (D / 64 each).  MQ = 1 is the
-// single-query case (fewer registers), MQ = kDecMaxQ takes 2..8 queries.
-template <typename T, int D, int MQ, bool LIST>
+// buffer, and for P.V the lanes own output dimensions (D / 64 each).  For 2..8 queries
+// (one: decode_one_kernel).
+template <typename T, int D, bool LIST>
 __global__ __launch_bounds__(256) void decode_kernel(const DecK a) {
+  constexpr int MQ = kDecMaxQ;
   constexpr int ESZ = sizeof(T);
   constexpr int RB = D * ESZ;     // row bytes
   constexpr int NC = RB / 16;     // 16-byte chunks per row
@@ -153,7 +176,7 @@ __global__ __launch_bounds__(256) void decode_kernel(const DecK a) {
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int split = blockIdx.x;
   const int64_t bh = blockIdx.y;
-  const int nq = MQ == 1 ? 1 : a.nq;
+  const int nq = a.nq;
 
   for (int u = tid; u < nq * NC; u += 256) {
     const int i = u / NC, cc = u - (u / NC) * NC;
@@ -174,22 +197,7 @@ __global__ __launch_bounds__(256) void decode_kernel(const DecK a) {
   const char* knew = a.n_new ? a.k_new + bh * a.new_sb : nullptr;
   const char* vnew = a.n_new ? a.v_new + bh * a.new_sb : nullptr;
 
-  // The appended rows this work-group owns (entry e of this class's segment in one of its
-  // groups) go to the cache: thread u copies 16-byte unit u % NC of the K (u < NC) or V
-  // row.  Nothing in this launch reads them back from the cache: the keys' lanes below
-  // take them from k_new / v_new.
-  for (int64_t j = 0; j < a.n_new; ++j) {
-    const int64_t t = a.new_pos0 + j;
-    const int64_t e = t / a.s;
-    const int64_t ncls = t - e * a.s;
-    if ((ncls * a.groups + (e >> 8)) % a.n_split != split) continue;
-    if (tid < 2 * NC) {
-      const int uu = tid % NC;
-      const char* src = (tid < NC ? knew : vnew) + j * a.new_sn + 16 * uu;
-      char* dst = (tid < NC ? a.k : a.v) + (bh * a.c_sb + ncls * a.Q * a.c_sn) * ESZ + e * rowb + 16 * uu;
-      *reinterpret_cast<du4*>(dst) = *reinterpret_cast<const du4*>(src);
-    }
-  }
+  copy_new_rows<NC>(a, bh, split, tid, rowb, knew, vnew, ESZ);
 
   float m[MQ], lsum[MQ], o[MQ][DPL];
 #pragma unroll
@@ -456,6 +464,217 @@ __global__ __launch_bounds__(256) void decode_kernel(const DecK a) {
   }
 }
 
+// x summed over the G lanes of each aligned group of G, the same value in all of them.
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {
+  const int y = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true);
+  return x + __builtin_bit_cast(float, y);
+}
+template <int G>
+__device__ __forceinline__ float group_sum(float x) {
+  static_assert(G == 8 || G == 16, "a row's lanes");
+  if constexpr (G == 16) x = dpp_add<0x140>(x);  // row_mirror
+  x = dpp_add<0x141>(x);                         // row_half_mirror
+  x = dpp_add<0x4e>(x);                          // quad_perm [2, 3, 0, 1]
+  return dpp_add<0xb1>(x);                       // quad_perm [1, 0, 3, 2]
+}
+
+// One query row.  Bound by the cache's bytes (K and V of the live keys, each read once),
+// so the kernel is built to keep memory busy: a row is read by the RB / 16 lanes of a group,
+// 16 bytes each (whole lines per instruction), K and V of a batch of 8 rows per group straight
+// into registers, and 16 waves per CU (two work-groups of 8) have their batches in flight
+// at different times.  The dot product is reduced over the group by DPP; the probability is
+// then in the lanes that hold the row's V, which keep their own running maximum, sum and output
+// and meet only at the end.  The live keys are listed as in decode_kernel, in a ring of 128
+// entries per wave; the ring starts a 64-key block at another place in neighbouring waves,
+// or all of them read the same part of a 16-KiB block at a time, which is the same channels'
+// in every head (110 -> 105 us in the first case below, 97 -> 88 with the next), with
+// non-temporal loads (a cached row is used once), and K's loads ahead of V's (88 -> 86).
+// Against decode_kernel, whose lanes read a K row each, wait for V in LDS and load nothing
+// meanwhile (us, both kernels of a call; bf16, D = 128): 256 heads x 3977 keys, causal 97.5 ->
+// 85.1 (5.4 -> 6.1 TB/s), 200 x 4100 106.7 -> 76.2, 32 x 65000 193 -> 162, 32 x 16011 51.2 ->
+// 49.1, band-256 | lattice-16 in its basis at 32 x 16011 21.2 -> 16.4, window 300 at 64 x 3977
+// 16.8 -> 14.1, D = 64 at 256 x 3977 51.4 -> 48.2; batches of 4 rows are as fast at the
+// largest and up to 1 us slower at the smallest, of 16 rows slower throughout.
+template <typename T, int D>
+__global__ __launch_bounds__(64 * kOneWaves) __attribute__((amdgpu_waves_per_eu(4)))
+void decode_one_kernel(const DecK a) {
+  constexpr int ESZ = sizeof(T);
+  constexpr int RB = D * ESZ;
+  constexpr int NC = RB / 16;    // lanes of a row
+  constexpr int RPI = 64 / NC;   // rows per load instruction
+  constexpr int NI = 8;          // rows per group and batch
+  constexpr int B = NI * RPI;    // rows per batch: 32 or 64
+  constexpr int DPL = 16 / ESZ;  // output dimensions per lane
+  __shared__ __attribute__((aligned(16))) float red_o[kOneWaves][D];
+  __shared__ float red_m[kOneWaves];
+  __shared__ float red_l[kOneWaves];
+  __shared__ int32_t kl_row[kOneWaves][128];
+  __shared__ pa_term terms_s[PA_MAX_TERMS];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int split = blockIdx.x;
+  const int64_t bh = blockIdx.y;
+  const int unit = lane % NC, sub = lane / NC;
+  const uint32_t n_groups = (uint32_t)(a.s * a.groups);
+  const int64_t rowb = a.c_sn * ESZ;
+  const char* knew = a.n_new ? a.k_new + bh * a.new_sb : nullptr;
+  const char* vnew = a.n_new ? a.v_new + bh * a.new_sb : nullptr;
+#pragma unroll
+  for (int i = 0; i < PA_MAX_TERMS; ++i)  // constant indices into the argument block
+    if (tid == i) terms_s[i] = a.pred.terms[i];
+  copy_new_rows<NC>(a, bh, split, tid, rowb, knew, vnew, ESZ);
+
+  const du4 q = *reinterpret_cast<const du4*>(a.q + bh * a.q_sb * ESZ + 16 * unit);
+  const char* kh = a.k + bh * a.c_sb * ESZ + 16 * unit;
+  const char* vh = a.v + bh * a.c_sb * ESZ + 16 * unit;
+
+  __syncthreads();
+
+  float m = -1e30f, lsum = 0.f, o[DPL];  // (finite: exp2(m - m_new) is 0, never NaN)
+#pragma unroll
+  for (int d = 0; d < DPL; ++d) o[d] = 0.f;
+
+  int head = 0, nlist = 0;  // the ring's first entry and length (at most B - 1 + 64)
+  uint32_t g = (uint32_t)split + (uint32_t)(w >> 2) * (uint32_t)a.n_split;
+  // the key of its 64 that lane 0 stands for, another batch's in neighbouring waves
+  const int rot = ((w + split + (int)bh) * B) & 63;
+  struct Batch {
+    du4 k[NI], v[NI];
+    int n;
+  };
+  // the next batch's rows, their loads in flight on return; false: none left
+  auto load = [&](Batch& t) __attribute__((always_inline)) -> bool {
+    while (nlist < B && g < n_groups) {
+      const int cls = (int)(g / (uint32_t)a.groups);
+      const int64_t b0 = (int64_t)(g - (uint32_t)cls * (uint32_t)a.groups) * 256 + 64 * (w & 3);
+      // (entries of the class; positions are below 2^31)
+      const int64_t i1 = a.length > cls ? (uint32_t)(a.length - 1 - cls) / (uint32_t)a.s + 1 : 0;
+      g += (kOneWaves / 4) * (uint32_t)a.n_split;
+      if (b0 >= i1) continue;
+      const int64_t idx = b0 + ((lane + rot) & 63);
+      const int32_t pos = (int32_t)(idx * a.s + cls);  // original position of this lane's key
+      const bool live = idx < i1 && pred_live_rolled(terms_s, a.pred.n_include, a.pred.n_exclude, (int32_t)a.qpos0,
+                                                      pos, a.pred.dense_bits, a.pred.dense_words);
+      const uint64_t any = __ballot(live);
+      if (live) {
+        const int at = head + nlist + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(any >> 32),
+                                                                     __builtin_amdgcn_mbcnt_lo((uint32_t)any, 0u));
+        const int64_t jn = (int64_t)pos - a.new_pos0;
+        kl_row[w][at & 127] = (jn >= 0 && jn < a.n_new) ? (int32_t)(-1 - jn) : (int32_t)(cls * a.Q + idx);
+      }
+      nlist += (int)__builtin_popcountll(any);
+    }
+    const int n = nlist < B ? nlist : B;
+    t.n = n;
+    if (n == 0) return false;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the list's entries are written
+    auto entry = [&](int e) { return kl_row[w][(head + (e < n ? e : 0)) & 127]; };  // (past n: the first again)
+    if (a.n_new && __ballot(entry(lane) < 0) != 0ull) {
+      // an appended token's row among them
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int32_t code = entry(i * RPI + sub);
+        const int64_t off = code < 0 ? (int64_t)(-1 - code) * a.new_sn + 16 * unit : (int64_t)code * rowb;
+        t.k[i] = *reinterpret_cast<const du4*>((code < 0 ? knew : kh) + off);
+        t.v[i] = *reinterpret_cast<const du4*>((code < 0 ? vnew : vh) + off);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        t.k[i] = __builtin_nontemporal_load(reinterpret_cast<const du4*>(kh + (int64_t)entry(i * RPI + sub) * rowb));
+      asm volatile("" ::: "memory");  // (K's loads first: the scores need nothing else)
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        t.v[i] = __builtin_nontemporal_load(reinterpret_cast<const du4*>(vh + (int64_t)entry(i * RPI + sub) * rowb));
+    }
+    asm volatile("" ::: "memory");  // the entries are read before the next are written
+    head += n;
+    nlist -= n;
+    return true;
+  };
+  auto consume = [&](Batch& t) __attribute__((always_inline)) {
+    float x[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x[i] = group_sum<NC>(Dec<T>::dot16(t.k[i], q, 0.f)) * a.c;
+    if (t.n < B) {
+      // rows past the list: no probability, and no value that 0 would not take out
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+        if (i * RPI + sub >= t.n) {
+          x[i] = -INFINITY;
+          t.v[i] = du4{0u, 0u, 0u, 0u};
+        }
+    }
+    float mn = m;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) mn = fmaxf(mn, x[i]);
+    const float alpha = exp2f(m - mn);
+    m = mn;
+    lsum *= alpha;
+#pragma unroll
+    for (int d = 0; d < DPL; ++d) o[d] *= alpha;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const float p = __builtin_amdgcn_exp2f(x[i] - mn);
+      lsum += p;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint32_t vw = t.v[i][c];
+        if constexpr (ESZ == 4) {
+          o[c] = __builtin_fmaf(p, Dec<T>::lo(vw), o[c]);
+        } else {
+          o[2 * c] = __builtin_fmaf(p, Dec<T>::lo(vw), o[2 * c]);
+          o[2 * c + 1] = __builtin_fmaf(p, Dec<T>::hi(vw), o[2 * c + 1]);
+        }
+      }
+    }
+  };
+  Batch t;
+  while (load(t)) consume(t);
+
+  // the groups' partials, then the waves'
+  float M = m;
+#pragma unroll
+  for (int h = NC; h < 64; h <<= 1) M = fmaxf(M, __shfl_xor(M, h));
+  const float f = exp2f(m - M);
+  lsum *= f;
+#pragma unroll
+  for (int d = 0; d < DPL; ++d) o[d] *= f;
+#pragma unroll
+  for (int h = NC; h < 64; h <<= 1) {
+    lsum += __shfl_xor(lsum, h);
+#pragma unroll
+    for (int d = 0; d < DPL; ++d) o[d] += __shfl_xor(o[d], h);
+  }
+  if (lane < NC) {
+#pragma unroll
+    for (int d = 0; d < DPL; ++d) red_o[w][lane * DPL + d] = o[d];
+  }
+  if (lane == 0) {
+    red_m[w] = M;
+    red_l[w] = lsum;
+  }
+  __syncthreads();
+  if (tid < D) {
+    float MM = red_m[0];
+#pragma unroll
+    for (int ww = 1; ww < kOneWaves; ++ww) MM = fmaxf(MM, red_m[ww]);
+    float L = 0.f, acc = 0.f;
+#pragma unroll
+    for (int ww = 0; ww < kOneWaves; ++ww) {
+      const float fw = exp2f(red_m[ww] - MM);
+      L += fw * red_l[ww];
+      acc += fw * red_o[ww][tid];
+    }
+    const int64_t row = bh * a.n_split + split;
+    a.o_part[row * D + tid] = acc * (L > 0.f ? 1.f / L : 0.f);
+    if (tid == 0) a.lse_part[row] = L > 0.f ? (MM + log2f(L)) * 0.69314718055994530942f : -INFINITY;
+  }
+}
+
 // o[bh, i] = sum_s exp(lse_s - M) o_s / sum_s exp(lse_s - M) over the splits; a row
 // whose every partial is empty gives 0 and lse -inf.  One work-group per (bh, i): the
 // weights are computed once into LDS, then 256 / D groups of D threads share the splits.
@@ -608,22 +827,19 @@ int check_decode(const pa_decode_args* x) {
   return PA_OK;
 }
 
-// The identity basis takes the kernel's key list (live keys spread thinly over many
+// Several queries: the identity basis takes the kernel's key list (live keys spread thinly over many
 // blocks); a residue basis, whose relabelling gathers the live keys into few full blocks,
 // takes block by block.
 template <typename T, int D>
 int launch_decode(const DecK& k, int64_t BH, hipStream_t s) {
   const dim3 grid((unsigned)k.n_split, (unsigned)BH);
   if (k.nq == 1) {
-    if (k.s == 1)
-      hipLaunchKernelGGL((decode_kernel<T, D, 1, true>), grid, dim3(256), 0, s, k);
-    else
-      hipLaunchKernelGGL((decode_kernel<T, D, 1, false>), grid, dim3(256), 0, s, k);
+    hipLaunchKernelGGL((decode_one_kernel<T, D>), grid, dim3(64 * kOneWaves), 0, s, k);
   } else {
     if (k.s == 1)
-      hipLaunchKernelGGL((decode_kernel<T, D, kDecMaxQ, true>), grid, dim3(256), 0, s, k);
+      hipLaunchKernelGGL((decode_kernel<T, D, true>), grid, dim3(256), 0, s, k);
     else
-      hipLaunchKernelGGL((decode_kernel<T, D, kDecMaxQ, false>), grid, dim3(256), 0, s, k);
+      hipLaunchKernelGGL((decode_kernel<T, D, false>), grid, dim3(256), 0, s, k);
   }
   PA_LAUNCH_CHECK("decode_kernel");
   return PA_OK;

@@ -88,6 +88,27 @@ def test_decode_other_dtypes_and_earlier_queries(gpu, dtype):
         check_close(out, want, dtype, f"decode {dtype} qpos0={qpos0} nq={nq} L={L}")
 
 
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.float16, 64), (torch.float32, 64)])
+@pytest.mark.parametrize("residue", [0, 4])
+def test_single_query_at_the_edges_of_a_batch(gpu, residue, dtype, D):
+    """One query row over lengths around the 32 or 64 keys of a wave's batch, its 64-key block
+    and a 256-key group, with the newest token appended by the call and rows past the length
+    that no result may touch (infinities)."""
+    BH, cap = 3, 768
+    q, k, v = make_qkv(BH, cap, D, dtype, seed=D + residue)
+    for L in (1, 2, 31, 32, 33, 63, 64, 65, 97, 128, 255, 257, 513, 767):
+        cache = pdec.KVCache(BH, cap, D, dtype, residue, gpu)
+        cache.k.fill_(float("inf"))
+        cache.v.fill_(float("inf"))
+        if L > 1:
+            cache.append(k[:, :L - 1].to(gpu), v[:, :L - 1].to(gpu))
+        out = cache.attend(q[:, L - 1:L].to(gpu), numpy_mask("causal"), k_new=k[:, L - 1:L].to(gpu),
+                           v_new=v[:, L - 1:L].to(gpu))
+        want, _ = oatt.dense_attention(as64(q[:, L - 1:L]), as64(k[:, :L]), as64(v[:, :L]),
+                                       lambda r0, r1: np.ones((r1 - r0, L), dtype=bool))
+        check_close(out, want, dtype, f"single query s={residue} D={D} L={L}")
+
+
 def test_dead_queries_and_empty_cache(gpu):
     BH, cap, D = 2, 512, 128
     q, k, v = make_qkv(BH, cap, D, torch.bfloat16, seed=2)
