@@ -39,7 +39,7 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _lib, registry
 from .index import STREAM_TILES, stream_arrays_for, wave_bits_for
 from .spec import DeviceMask, MaskSpec, as_perm_tensor
 
@@ -58,14 +58,12 @@ def _assert_kinds_match():
         raise RuntimeError(f"kind constants diverged: triton_attn={mine} masks_gpu={theirs}")
 
 
-_KINDS_CHECKED = False
-
-
-def _check_kinds_once():
-    """The constants of both modules are fixed once imported: compared at the first call."""
-    global _KINDS_CHECKED
-    _assert_kinds_match()
-    _KINDS_CHECKED = True
+def _check_kinds():
+    """The same at each call, without building the message's tables."""
+    if (CAUSAL, WINDOW, DILATED, LOCAL_STRIDED, TWOBAND, SINKS, PREFIX_LM) != (
+            registry.CAUSAL, registry.WINDOW, registry.DILATED, registry.LOCAL_STRIDED, registry.TWOBAND,
+            registry.SINKS, registry.PREFIX_LM):
+        _assert_kinds_match()
 
 
 def _rows3(t, name):
@@ -130,8 +128,7 @@ def prepare(q, k, v, kv_idx, kv_num, kv_partial, kind, p0, p1, p2, BQ, A, scale=
     BH, N, D = q.shape
     if perm_kv is None:
         perm_kv = perm_q
-    if not _KINDS_CHECKED:
-        _check_kinds_once()
+    _check_kinds()
     assert N % BQ == 0 and N % A == 0, "cost model and kernel both assume this"
     assert k.shape == v.shape == q.shape
     if int(gather_mult) < 1:
