@@ -290,6 +290,15 @@ void attn_narrow_kernel(const AttnK a, int units, int groups) {
     }
     asm volatile("" ::"v"(r_tile), "v"(r_code), "v"(r_boff));
   };
+  // A list of an odd number of segments: its last step's second one is past it, with no
+  // pairs and V rows that are the first one's again, and 0 times an infinity is no 0.
+  auto clear_past = [&](int S) __attribute__((always_inline)) {
+    if (n_seg & 1) {
+#pragma unroll
+      for (int i = 0; i < R::NI; ++i)
+        *(lds_u4w*)((lds_char_t*)ring_s + w * 2 * STAGE + S * STAGE + SEG + i * 1024 + 16 * lane) = u32x4{0u, 0u, 0u, 0u};
+    }
+  };
   if (n_steps > 0) {
     load_raw(0);
     prefetch(0, 0, s0, d0);
@@ -300,11 +309,15 @@ void attn_narrow_kernel(const AttnK a, int units, int groups) {
     prefetch(j + 1, 1, s1, d1);
     compute(0, s0, d0);
     arrive(d1);
-    if (j + 2 < n_steps) prefetch(j + 2, 0, s0, d0);
+    if (j + 2 < n_steps)
+      prefetch(j + 2, 0, s0, d0);
+    else
+      clear_past(1);
     compute(1, s1, d1);
   }
   if (j < n_steps) {
     arrive(d0);
+    clear_past(0);
     compute(0, s0, d0);
   }
 

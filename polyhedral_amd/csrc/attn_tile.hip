@@ -240,8 +240,9 @@ void attn_tile_kernel(const AttnK a) {
   for (int i = 0; i < NDB; ++i) acc[i] = f32x16{0};
   float m_run = kSentinel, l_part = 0.f;
 
-  // A step in stage SC.  FULL: every pair of it live for this wave (no masking, no branch).
-  auto compute = [&](auto SC, auto FULL, const Step& s, const uint32_t* wd, int col0, int col1)
+  // A step in stage SC, with `rest` segments of the list left from its first on.  FULL: every
+  // pair of it live for this wave (no masking, no branch).
+  auto compute = [&](auto SC, auto FULL, const Step& s, const uint32_t* wd, int rest, int col0, int col1)
                      __attribute__((always_inline)) {
     constexpr int SO = decltype(SC)::value * STAGE;
     constexpr bool ALL = decltype(FULL)::value;
@@ -315,6 +316,9 @@ void attn_tile_kernel(const AttnK a) {
       if (!ALL && ((s.live >> (2 * lb)) & 3u) == 0u) continue;
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
+        // (a segment past the list has no pairs, and 0 times its V rows, which are another
+        // segment's, is no 0 where they hold an infinity)
+        if (!ALL && c == 1 && 2 * lb + 1 >= rest) continue;
         f32x8 pv;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -374,10 +378,11 @@ void attn_tile_kernel(const AttnK a) {
       col1 = __shfl(c_col, s.u4 + 2 + (m >> 4)) + (m & 15);
     }
     if (j + 1 < n_steps) prefetch(j + 1, S ^ 1);
+    const int rest = n_seg - 4 * (j * KG + kg);
     if (s.full == 15u)
-      compute(SC, std::true_type{}, s, wd, col0, col1);
+      compute(SC, std::true_type{}, s, wd, rest, col0, col1);
     else if (s.live != 0u)
-      compute(SC, std::false_type{}, s, wd, col0, col1);
+      compute(SC, std::false_type{}, s, wd, rest, col0, col1);
   };
   if (n_steps > 0) {
     load_raw(0);
