@@ -32,8 +32,12 @@ streaming kernel whenever its preconditions hold and the index carries its array
 
 The HIP kernels that serve the call: the streaming kernel (f16 / bf16, D = 128, BQ = 128,
 A in 16, 32, 64) moves K and V into LDS by DMA and masks from bitmaps; the tile kernels
-(f16 / bf16, "auto" only) do so from the plain lists, with or without bitmaps; the wave-split kernel takes small float32 grids; the general kernel takes every
-other shape and dtype and can evaluate the predicate itself.
+(f16 / bf16, "auto" only) do so from the plain lists, with or without bitmaps; the
+wave-split kernel takes small float32 grids; the general kernel takes every other shape and
+dtype and can evaluate the predicate itself.
+
+NaN and infinities in q, k and v: the tile kernels give NaN and infinities in the same
+places as the general kernel, a row with a NaN (or +inf) live score being NaN with lse -inf.
 """
 import ctypes
 

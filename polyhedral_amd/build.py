@@ -45,11 +45,11 @@ def _torch_lib():
     return pathlib.Path(spec.origin).parent / "lib"
 
 
-# per-source additions: the streaming, tile and narrow kernels compute no NaN on purpose (masked scores
+# per-source additions: the streaming kernel computes no NaN on purpose (masked scores
 # are -inf, never NaN), so fmax needs no NaN-quieting instructions
-EXTRA_FLAGS = {"attn_stream.hip": ["-fno-honor-nans", "-Wno-inline-asm"],
-               "attn_tile.hip": ["-fno-honor-nans", "-Wno-inline-asm"],
-               "attn_narrow.hip": ["-fno-honor-nans", "-Wno-inline-asm"], "bwd.hip": ["-Wno-inline-asm"], "decode.hip": ["-Wno-inline-asm"]}
+EXTRA_FLAGS = {"attn_stream.hip": ["-fno-honor-nans", "-Wno-inline-asm"], "attn_tile.hip": ["-Wno-inline-asm"],
+               "attn_narrow.hip": ["-Wno-inline-asm"], "bwd.hip": ["-Wno-inline-asm"],
+               "decode.hip": ["-Wno-inline-asm"]}
 
 
 def _compile(src, hipcc):

@@ -43,7 +43,7 @@ __device__ __forceinline__ f32x4 mma16x32(typename Mma<T>::frag a, typename Mma<
 // max / sum over the four lanes l % 16 + 16 g that hold one query row
 __device__ __forceinline__ float quad_max(float x) {
   const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
-  return row_max(fmaxf(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1])));
+  return row_nan_max(nan_max(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1])));
 }
 __device__ __forceinline__ float quad_sum(float x) {
   const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
@@ -247,9 +247,9 @@ void attn_narrow_kernel(const AttnK a, int units, int groups) {
           if (!((word >> i) & 1u)) x[t][i] = -INFINITY;
       }
     }
-    const float mx = quad_max(fmaxf(fmaxf(fmaxf(x[0][0], x[0][1]), fmaxf(x[0][2], x[0][3])),
-                                    fmaxf(fmaxf(x[1][0], x[1][1]), fmaxf(x[1][2], x[1][3]))));
-    const float m_new = fmaxf(m_run, mx * a.c);
+    const float mx = quad_max(nan_max(nan_max(nan_max(x[0][0], x[0][1]), nan_max(x[0][2], x[0][3])),
+                                      nan_max(nan_max(x[1][0], x[1][1]), nan_max(x[1][2], x[1][3]))));
+    const float m_new = nan_max(m_run, mx * a.c);
     if (__ballot(m_new > m_run + kLazy) != 0ull) {
       const float alpha = exp2f(m_run - m_new);
       m_run = m_new;

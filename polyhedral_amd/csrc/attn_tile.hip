@@ -277,7 +277,7 @@ void attn_tile_kernel(const AttnK a) {
 #pragma unroll
       for (int lb = 0; lb < 2; ++lb)
 #pragma unroll
-        for (int i = 0; i < 16; i += 2) mx = fmaxf(mx, fmaxf(sc[lb][i], sc[lb][i + 1]));
+        for (int i = 0; i < 16; i += 2) mx = nan_max(mx, nan_max(sc[lb][i], sc[lb][i + 1]));
     } else {
 #pragma unroll
       for (int lb = 0; lb < 2; ++lb) {
@@ -298,11 +298,11 @@ void attn_tile_kernel(const AttnK a) {
           }
         }
 #pragma unroll
-        for (int i = 0; i < 16; i += 2) mx = fmaxf(mx, fmaxf(x[i], x[i + 1]));
+        for (int i = 0; i < 16; i += 2) mx = nan_max(mx, nan_max(x[i], x[i + 1]));
         sc[lb] = x;
       }
     }
-    const float m_new = fmaxf(m_run, row_max(mx) * a.c);
+    const float m_new = nan_max(m_run, row_nan_max(mx) * a.c);
     if (__ballot(m_new > m_run + kLazy) != 0ull) {
       const float alpha = exp2f(m_run - m_new);
       m_run = m_new;

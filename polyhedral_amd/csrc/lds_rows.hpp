@@ -76,6 +76,16 @@ __device__ __forceinline__ TileReads<D> tile_reads(lds_cptr lds, int lane) {
   return t;
 }
 
+// Maximum that gives NaN when either side is NaN: one instruction (v_maximum3_f32) on scores
+// straight from an MFMA, where fmaxf, which gives the other side, needs one more per score to
+// quiet signalling NaNs.  A row with a NaN score is NaN either way, by its probabilities.
+__device__ __forceinline__ float nan_max(float x, float y) { return __builtin_elementwise_maximum(x, y); }
+// Over lanes l and l ^ 32, as row_max.
+__device__ __forceinline__ float row_nan_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), false, false);
+  return nan_max(__builtin_bit_cast(float, (int)r[0]), __builtin_bit_cast(float, (int)r[1]));
+}
+
 // A operand X^T of 16 rows of a staged tile at byte offset `off` (stage + tile + first row):
 // the transposed product's fragment for block db of D.
 template <typename T, int D>

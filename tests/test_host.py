@@ -137,3 +137,11 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(root, "bench.py"), "--gpus", "2"], capture_output=True,
                        text=True, timeout=300)
     assert r.returncode == 2 and "one GPU" in r.stderr
+
+
+def test_only_the_streaming_kernel_is_compiled_without_nans():
+    """A row whose sum is NaN must compare as NaN in the kernels' epilogues (l > 0 is false)."""
+    from polyhedral_amd import build
+    flagged = {src for src, flags in build.EXTRA_FLAGS.items() if any("nans" in f or "fast" in f for f in flags)}
+    assert flagged == {"attn_stream.hip"}
+    assert not any("nans" in f or "fast" in f for f in build.HIP_FLAGS)
