@@ -80,7 +80,7 @@ def _term_struct(include, exclude):
     m = _lib.PaMask()
     m.n_include, m.n_exclude = len(include), len(exclude)
     for i, t in enumerate(include + exclude):
-        m.terms[i] = _lib.PaTerm(*[int(x) for x in t])
+        m.terms[i] = _lib.PaTerm(*t)
     return m
 
 
@@ -122,8 +122,9 @@ class DeviceMask:
     _keep: list = field(default_factory=list)
 
     def struct(self):
-        m = _lib.PaMask.from_buffer_copy(_term_struct(tuple(map(tuple, self.spec.include)),
-                                                      tuple(map(tuple, self.spec.exclude))))
+        # (by value: a parameter may be any integer, also one that has no hash or hashes by identity)
+        m = _lib.PaMask.from_buffer_copy(_term_struct(tuple([tuple(map(int, t)) for t in self.spec.include]),
+                                                      tuple([tuple(map(int, t)) for t in self.spec.exclude])))
         m.perm_q = _lib.address(self.perm_q)
         m.perm_kv = _lib.address(self.perm_kv)
         if self.dense_bits is not None:

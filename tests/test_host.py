@@ -145,3 +145,19 @@ def test_only_the_streaming_kernel_is_compiled_without_nans():
     flagged = {src for src, flags in build.EXTRA_FLAGS.items() if any("nans" in f or "fast" in f for f in flags)}
     assert flagged == {"attn_stream.hip"}
     assert not any("nans" in f or "fast" in f for f in build.HIP_FLAGS)
+
+
+def test_mask_struct_reads_its_parameters_at_each_call():
+    """Term parameters may be any integers: 0-d arrays (which have no hash) and 0-d tensors
+    (whose hash is their identity, and which may change in place)."""
+    import torch
+    from polyhedral_amd.spec import DeviceMask, MaskSpec
+    WINDOW, SINKS = 1, 5
+    m = DeviceMask(MaskSpec(((WINDOW, np.array(100), 0, 0),))).struct()
+    assert (m.n_include, m.terms[0].kind, m.terms[0].p0) == (1, WINDOW, 100)
+    w = torch.tensor(64)
+    dm = DeviceMask(MaskSpec(((SINKS, w, 4, 0),), ([WINDOW, 8, 0, 0],)))
+    assert dm.struct().terms[0].p0 == 64
+    w.fill_(65)
+    m = dm.struct()
+    assert m.terms[0].p0 == 65 and (m.n_exclude, m.terms[1].p0) == (1, 8)
