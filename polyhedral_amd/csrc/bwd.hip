@@ -306,12 +306,14 @@ void bwd_dkdv_kernel(const BwdK a) {
   dma_offsets<D>(dvoff, pitch, lane);
   // Query block qb into stage S: the rows of Q and dO by every wave, rowsum(dO O) by wave 1,
   // a partial tile's bitmap (bo >= 0) by waves 2 and 3 or, without bitmaps, the original row
-  // numbers by wave 2.  The lse goes through wave 0's registers (lse_n, written as the
-  // exponent offset by put_lse once it has arrived).
+  // numbers by wave 2.  The lse goes through registers (lse_n): once it has arrived, put_lse
+  // writes it as the exponent offset (wave 0) and keeps which of the wave's 32 rows have no
+  // weight (lse = -inf: P is 0 also where their scores are NaN).
   float lse_n = 0.f;
+  uint32_t dead_n = 0u;
   auto dma = [&](int qb, int bo, int S) __attribute__((always_inline)) {
     const int64_t r0 = mem_row(a, qb * kBT);
-    if (w == 0) lse_n = hlse[r0 + rs * lane];
+    lse_n = hlse[r0 + rs * lane];
     dma_tiles<D>(lds0 + S * TL::STAGE, hq, hdo, pitch, r0 * rowb, w, dvoff);
     const uint32_t mv = lds0 + TL::VEC_OFF + S * TL::VEC;
     if (w == 1) dma_x1(mv + 256, hdvec + r0 * 4, 4u * rs * lane);
@@ -324,6 +326,7 @@ void bwd_dkdv_kernel(const BwdK a) {
   };
   auto put_lse = [&](int S) __attribute__((always_inline)) {
     if (w == 0) *(lds_fw*)((lds_char_t*)gsm + TL::VEC_OFF + S * TL::VEC + 4 * lane) = neg_lse2(lse_n);
+    dead_n = (uint32_t)(__ballot(lse_n == -INFINITY) >> (32 * qh));
   };
 
   const TileReads<D> rd = tile_reads<D>(lds + 32 * qh * TL::ROW, lane);
@@ -338,7 +341,7 @@ void bwd_dkdv_kernel(const BwdK a) {
 #pragma unroll
   for (int i = 0; i < NDB; ++i) dkt[i] = dvt[i] = f32x16{0};
 
-  auto tile = [&](auto SC, bool partial, int qb) __attribute__((always_inline)) {
+  auto tile = [&](auto SC, bool partial, int qb, uint32_t dead) __attribute__((always_inline)) {
     constexpr int S = decltype(SC)::value;
     constexpr int SO = S * TL::STAGE;
     // element i of the lane: query row 32 qh + 8 (i / 4) + 4 G + i % 4, key `key`
@@ -359,10 +362,13 @@ void bwd_dkdv_kernel(const BwdK a) {
       for (int e = 0; e < 4; ++e)
         s[4 * j + e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[4 * j + e], a.c, nl[e]));
     }
-    if (partial) {
-      uint32_t word;
+    // (dead rows with the bitmap where there is one, apart where the mask is evaluated: the
+    // other way round costs 2% at D = 128 and spills 8 registers)
+    if (partial || (BITS && dead != 0u)) {
+      uint32_t word = ~0u;
       if constexpr (BITS) {
-        word = *(lds_u32*)(lds + TL::VEC_OFF + S * TL::VEC + 512 + (32 * kh + m) * 8 + 4 * qh);
+        if (partial) word = *(lds_u32*)(lds + TL::VEC_OFF + S * TL::VEC + 512 + (32 * kh + m) * 8 + 4 * qh);
+        word &= ~dead;
       } else {
         lds_i32* qo = (lds_i32*)(lds + TL::VEC_OFF + S * TL::VEC + 512 + 128 * qh);
         word = live_word(a, terms_s, G, [&](int b) { return hperm ? qo[b] : qb * kBT + 32 * qh + b; },
@@ -370,6 +376,7 @@ void bwd_dkdv_kernel(const BwdK a) {
       }
       mask16(s, word, G);
     }
+    if (!BITS && dead != 0u) mask16(s, ~dead, G);
     PA_FENCE();
     Frag pf[2], sf[2];
     to_frags<T>(s, pf);
@@ -431,11 +438,12 @@ void bwd_dkdv_kernel(const BwdK a) {
     __syncthreads();  // stage S is in; every wave is past stage S ^ 1
     if (t + NG < nl) dma(qb_n, bo_n, S ^ 1);
     const int qb = qb_c;
+    const uint32_t dead = dead_n;
     const bool partial = bo_c >= 0;
     qb_c = qb_n;
     bo_c = bo_n;
     if (t + 2 * NG < nl) tile_of(t + 2 * NG, qb_n, bo_n);
-    if (NG == 1 || t < nl) tile(SC, partial, qb);
+    if (NG == 1 || t < nl) tile(SC, partial, qb, dead);
     if (t + NG < nl) put_lse(S ^ 1);
   };
   // (every group takes every step: the last one may have no tile for it)
@@ -520,6 +528,8 @@ void bwd_dq_kernel(const BwdK a) {
   Frag qf[NKC], df[NKC];
   const float nl2 = neg_lse2(a.lse[bh * a.lse_sb + row_m]);
   const float dr = a.dvec[bh * a.lse_sb + row_m];
+  const bool dead = nl2 == -INFINITY;  // a row with no weight: P is 0 also where its scores are NaN
+  const bool any_dead = __ballot(dead) != 0ull;
   f32x16 dqt[NDB];
 #pragma unroll
   for (int i = 0; i < NDB; ++i) dqt[i] = f32x16{0};
@@ -547,6 +557,10 @@ void bwd_dq_kernel(const BwdK a) {
                          [&](int b) { return hperm ? ko[b] : kb * kBT + 32 * kh + b; });
       }
       mask16(s, word, G);
+    }
+    if (any_dead) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = dead ? 0.f : s[i];
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] *= dp[i] - dr;

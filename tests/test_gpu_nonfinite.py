@@ -1,9 +1,11 @@
 """What infinities and NaN in the inputs do: the f16 / bf16 kernels on plain block lists
-(pa_attn_fwd_tile) give them in the same places as the general kernel on the same arguments."""
+(pa_attn_fwd_tile) give them in the same places as the general kernel on the same arguments,
+and rows that the forward found no weight for stay out of the backward."""
 import pytest
 import torch
 
 from polyhedral_amd import attention as pattn
+from polyhedral_amd import backward
 from polyhedral_amd import index as pindex
 from polyhedral_amd.polyattn import masks as pm
 from tests.util import make_qkv
@@ -79,3 +81,32 @@ def test_same_places_as_the_general_kernel(gpu, D, dtype, BQ, A, inputs):
             # (P is rounded at another running maximum: at most 2 eps sum p |v|, and an ulp of the result's rounding)
             assert bool(((o1 - o2).abs() <= 2 * eps * big + 2 * eps * o1.abs()).all())
             assert float((l1 - l2).abs().max()) < 2e-5
+
+
+@pytest.mark.parametrize("bitmaps", [True, False])
+@pytest.mark.parametrize("BH", [2, 40])  # 16 work-groups of two groups of waves, 320 of one
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+def test_backward_rows_without_weight(gpu, D, dtype, BH, bitmaps):
+    """A row whose lse is -inf (no live key, or scores that are not finite: the forward gives
+    both) has P = 0 whatever its scores: dV of every key and dQ of every row are those of the
+    same row with finite values."""
+    N = 512
+    q, k, v = (x.to(gpu) for x in make_qkv(BH, N, D, dtype, seed=D))
+    o, do, _ = (x.to(gpu) for x in make_qkv(BH, N, D, dtype, seed=D + 1))
+    lse = torch.full((BH, N), 6.0, device=gpu)
+    rows = [0, 77, 200, 511]  # in partial tiles and in full ones
+    lse[:, rows] = -INF
+    o[:, rows] = 0
+    plan = backward.BackwardPlan(pm.Causal(), N, gpu, bitmaps=bitmaps)
+    dq, _, dv = plan.backward(q, k, v, o, lse, do)
+    assert bool(torch.isfinite(dq).all()) and bool(torch.isfinite(dv).all())
+    assert torch.count_nonzero(dq[:, rows]) == 0
+    for value in (NAN, INF):
+        bad = q.clone()
+        bad[:, rows, 3] = value
+        dq2, _, dv2 = plan.backward(bad, k, v, o, lse, do)
+        assert torch.equal(dv, dv2) and torch.equal(dq, dq2)
+    # the last key, which only the last row (without weight) sees
+    bad = k.clone()
+    bad[:, 511, 3] = INF
+    assert torch.equal(plan.backward(q, bad, v, o, lse, do)[2], dv)
