@@ -492,44 +492,55 @@ int launch_tile_t(const AttnK& a, hipStream_t s) {
 }
 
 // How many key groups a list is given and into how many pieces of 64 rows a block of 128 is
-// cut: small launches wait for their longest lists.  Measured (us; causal unless said), 128
-// rows by one key group / 128 rows by two / pieces of 64 rows by two / by four:
+// cut.  A second group halves what a launch of up to one work-group per CU waits for; beyond
+// that it pays where a few lists are much longer than the rest (uneven: a covering mask in
+// order), and costs where all are alike.  Measured (us; f16, lists of tiles with bitmaps / by
+// the predicate where two figures stand; w: a window), by one key group of 128 rows / two /
+// pieces of 64 rows by two / by four:
 //   D = 64, work-groups of 128 rows:
-//     64 (2 x 4096)   - / 50.5 / 41.8 / 33.2      128 (1 x 16384) - / 183 / 153 / 111
-//     128 (window 200, 4 x 4096) - / 10.7 / 9.3 / 9.3     128 (window 1024) - / 18.4 / 15.2 / 13.5
-//     256 (8 x 4096) 73.2 / 51.7 / 43.5 / 53.6    256 (4 x 8192) - / 91.6 / 76.2 / 96.7
-//     256 (32 x 1024) - / 21.1 / 22.1 / 30.2      256 (window 4096, 4 x 8192) - / 49.5 / 50.5 / 57.7
-//     384 (12 x 4096) 93.8 / 63.9 / 60.8 / 74.0   512 (16 x 4096) - / 64.4 / 72.2 / 94.3
-//   so four key groups and pieces up to 128 work-groups, which then fit one to a CU; up to
-//   384 two groups and pieces where the longest list covers most of the sequence (the lists
-//   then mostly differ, and a CU takes a long and a short piece) and is long enough to pay
-//   for staging it twice;
-//   D = 128: 64 (2 x 4096) - / 70.8 / 58.8, 128 (4 x 4096) - / 71.3 / 60.1, 128 (window 200)
+//     64 (causal, 2 x 4096)   - / 50.5 / 41.8 / 33.2      128 (causal, 1 x 16384) - / 183 / 153 / 111
+//     128 (w 200, 4 x 4096) - / 10.7 / 9.3 / 9.3     128 (w 1024) - / 18.4 / 15.2 / 13.5
+//     256 (causal, 8 x 4096) 73.2 / 51.7 / 43.5 / 53.6    256 (causal, 4 x 8192) - / 91.6 / 76.2 / 96.7
+//     256 (32 x 1024) - / 21.1 / 22.1 / 30.2      256 (w 4096, 4 x 8192) - / 49.5 / 50.5 / 57.7
+//     320 (w 200) 14.3 55.0 / 18.0 58.3 / 16.7 58.3 / 22.1 66.5, (w 2048) 46.4 68.4 / 41.7 56.3
+//     384 (causal, 12 x 4096) 93.8 / 63.9 / 60.8 / 74.0   512 (causal, 16 x 4096) - / 64.4 / 72.2 / 94.3
+//     512 (w 64) 11.0 27.3 / 15.1 36.3, (w 300) 16.5 51.7 / 20.8 70.8, (w 1536) 39.2 59.5 / 43.6 63.4,
+//     (lattice 8 in its basis) 37.1 48.9 / 46.7 61.5, (band and lattice 16 in the lattice's) 68.8 / 74.4
+//   so four key groups and pieces up to 128 work-groups, which then fit one to a CU; two groups
+//   up to 256, and on long lists a quarter more; up to 512 two groups on uneven lists, in
+//   pieces up to 384 (a CU takes a long and a short one);
+//   D = 128: 64 (2 x 4096) - / 70.8 / 58.8, 128 (4 x 4096) - / 71.3 / 60.1, 128 (w 200)
 //     - / 39.9 / 32.4, 160 (5 x 4096) - / 72.2 / 71.0, 160 (10 x 2048) - / 42.6 / 47.0, 256
 //     107 / 74.7 / 89.0 (one work-group of two groups per CU by its LDS).
 // Blocks of 64 rows, one key group / two / four:
 //   D = 64:  128 (8 x 1024) - / 18.4 / 16.9, 256 (8 x 2048) - / 26.6 / 22.6, 256 (4 x 4096) - /
-//     42.6 / 33.9, 512 (8 x 4096) 71.8 / 43.4 / 53.6, 2048 (window 1024) 85 / 105 / -;
-//   D = 128: 512 105 / 95, 2048 (window 1024) 172 / 227.
+//     42.6 / 33.9, 512 (8 x 4096) 71.8 / 43.4 / 53.6, 768 (w 128) 10.4 22.1 / 14.8 36.2, 1024 (w 300)
+//     15.7 36.9 / 19.0 51.2, 2048 (w 1024) 85 / 105 / -;
+//   D = 128: 512 (causal, 8 x 4096) 87.4 / 78.2, (causal, 16 x 2048) 60.8 / 38.6, (w 128) 13.1 24.4 /
+//     19.1 38.7, (w 1024) 37.2 48.1 / 40.2 59.6, (band and lattice 16 in the lattice's basis) 60.2 355
+//     / 83.4 460; 2048 (w 1024) 172 / 227.
 template <typename T, int D>
 int launch_tile_d(const AttnK& a, hipStream_t s) {
+  const int64_t wgs = a.total_wg, longest = a.pitch * a.A;
+  // (in a residue basis a covering mask's lists are about equally long)
+  const bool uneven = longest >= 2048 && 4 * longest >= 3 * (int64_t)a.N && !a.residue_s && !a.pred.perm_q;
   if constexpr (D == 64) {
     if (a.BQ == 64) {
-      if (a.total_wg <= 256) return launch_tile_t<T, D, 2, 4, 1>(a, s);
-      if (a.total_wg <= 1024) return launch_tile_t<T, D, 2, 2, 1>(a, s);
+      if (wgs <= 256) return launch_tile_t<T, D, 2, 4, 1>(a, s);
+      if (wgs <= 512 || (wgs <= 1024 && uneven)) return launch_tile_t<T, D, 2, 2, 1>(a, s);
       return launch_tile_t<T, D, 2, 1, 1>(a, s);
     }
-    if (a.total_wg <= 128) return launch_tile_t<T, D, 2, 4, 2>(a, s);
-    const int64_t longest = a.pitch * a.A;
-    if (a.total_wg <= 384 && longest >= 2048 && 4 * longest >= 3 * (int64_t)a.N) return launch_tile_t<T, D, 2, 2, 2>(a, s);
-    if (a.total_wg <= 512) return launch_tile_t<T, D, 4, 2, 1>(a, s);
+    if (wgs <= 128) return launch_tile_t<T, D, 2, 4, 2>(a, s);
+    if (wgs <= 384 && uneven) return launch_tile_t<T, D, 2, 2, 2>(a, s);
+    if (wgs <= 256 || (wgs <= 320 && longest >= 1536) || (wgs <= 512 && uneven))
+      return launch_tile_t<T, D, 4, 2, 1>(a, s);
   } else {
     if (a.BQ == 64) {
-      if (a.total_wg <= 512) return launch_tile_t<T, D, 2, 2, 1>(a, s);
+      if (wgs <= 256 || (wgs <= 512 && uneven)) return launch_tile_t<T, D, 2, 2, 1>(a, s);
       return launch_tile_t<T, D, 2, 1, 1>(a, s);
     }
-    if (a.total_wg <= 128) return launch_tile_t<T, D, 2, 2, 2>(a, s);
-    if (a.total_wg <= 256) return launch_tile_t<T, D, 4, 2, 1>(a, s);
+    if (wgs <= 128) return launch_tile_t<T, D, 2, 2, 2>(a, s);
+    if (wgs <= 256) return launch_tile_t<T, D, 4, 2, 1>(a, s);
   }
   return launch_tile_t<T, D, 4, 1, 1>(a, s);
 }

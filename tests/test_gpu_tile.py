@@ -67,6 +67,22 @@ def test_equals_general_kernel(gpu, name, D, dtype, BH, N, BQ, A, bitmaps):
           heads_desc=bitmaps)
 
 
+@pytest.mark.parametrize("name,D,BH,N", [
+    # work-groups of 128 / 64 rows, whether the lists are uneven (a covering mask in order, 2048 and longer)
+    ("causal", 128, 9, 2048),        # 144 / 288 uneven: two groups
+    ("window-128", 128, 9, 2048),    # 144 / 288: one group for 64 rows
+    ("causal", 64, 20, 2048),        # 320 / 640 uneven: pieces by two groups / two groups
+    ("causal", 64, 26, 2048),        # 416 / 832 uneven: two groups
+    ("window-128", 64, 20, 2048),    # 320 / 640: one group
+    ("causal", 64, 40, 1024),        # 320 / 640, covering but shorter than 2048: one group
+])
+@pytest.mark.parametrize("BQ,A", [(128, 32), (64, 64)])
+def test_groups_by_the_lists_evenness(gpu, name, D, BH, N, BQ, A):
+    q, k, v = (x.to(gpu) for x in make_qkv(BH, N, D, torch.float16, seed=BH + N))
+    lists, wave, bits = _built(numpy_mask(name), N, BQ, A, gpu)
+    _both(q, k, v, lists, triton_params(name), BQ, A, kv_wave_bits=wave, kv_bits=bits)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("BQ,A", [(128, 32), (64, 64), (32, 32), (16, 16)])
 def test_bases_strides_order_and_merge(gpu, BQ, A, D):
