@@ -110,36 +110,51 @@ __device__ __forceinline__ Verdict term_verdict(const pa_term& t, const Range& r
   }
 }
 
-// The whole predicate: live where an include term is and no exclude term is.
+// The whole predicate: live where an include term is and no exclude term is.  The terms come
+// from LDS in a rolled loop: unrolled over the argument block, the two uses below held 263
+// spilled scalars (118 now) beside the pairs' evaluation.  With that and with ranges taken by
+// shuffles, a build in a random permutation, where hardly a block is decided here, took 7 to
+// 12% longer than evaluating every pair alone (16x16 tiles, N = 16256, window 300: 1158 us
+// against 1043; now 1051).
 template <typename F>
-__device__ __forceinline__ Verdict pred_verdict(const Pred& p, const Range& r, F same) {
+__device__ __forceinline__ Verdict pred_verdict(const pa_term* terms, int n_include, int n_exclude, const Range& r,
+                                                F same) {
   Verdict inc = kDead, exc = kDead;
-  const int n = p.n_include + p.n_exclude;
-#pragma unroll
-  for (int i = 0; i < PA_MAX_TERMS; ++i) {  // (constant indices into the argument block)
-    if (i < n) {
-      const Verdict v = term_verdict(p.terms[i], r, same);
-      Verdict& to = i < p.n_include ? inc : exc;
-      if (v == kLive || to == kLive)
-        to = kLive;
-      else if (v == kMixed)
-        to = kMixed;
-    }
+#pragma unroll 1
+  for (int i = 0; i < n_include + n_exclude; ++i) {
+    pa_term t;  // (the same in every lane)
+    t.kind = __builtin_amdgcn_readfirstlane(terms[i].kind);
+    t.p0 = __builtin_amdgcn_readfirstlane(terms[i].p0);
+    t.p1 = __builtin_amdgcn_readfirstlane(terms[i].p1);
+    t.p2 = __builtin_amdgcn_readfirstlane(terms[i].p2);
+    const Verdict v = term_verdict(t, r, same);
+    Verdict& to = i < n_include ? inc : exc;
+    if (v == kLive || to == kLive)
+      to = kLive;
+    else if (v == kMixed)
+      to = kMixed;
   }
   if (inc == kDead || exc == kLive) return kDead;
   return (inc == kLive && exc == kDead) ? kLive : kMixed;
 }
 
+// Minimum over a wave, in every lane (cross-lane moves of the VALU: in a table basis it is
+// taken for every 64 columns, and shuffles through LDS wait for one another).
+template <int CTRL>
+__device__ __forceinline__ int32_t dpp_min(int32_t x) {
+  return min(x, __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ int32_t wave_min(int32_t x) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) x = min(x, __shfl_xor(x, o));
-  return x;
+  x = dpp_min<0x140>(x);  // row_mirror
+  x = dpp_min<0x141>(x);  // row_half_mirror
+  x = dpp_min<0x4e>(x);   // quad_perm [2, 3, 0, 1]
+  x = dpp_min<0xb1>(x);   // quad_perm [1, 0, 3, 2]
+  const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  x = min((int32_t)r[0], (int32_t)r[1]);
+  const auto h = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return min((int32_t)h[0], (int32_t)h[1]);
 }
-__device__ __forceinline__ int32_t wave_max_i(int32_t x) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) x = max(x, __shfl_xor(x, o));
-  return x;
-}
+__device__ __forceinline__ int32_t wave_max_i(int32_t x) { return ~wave_min(~x); }
 
 __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int32_t N, int32_t BQ,
                                                              int32_t A, uint32_t* __restrict__ codes,
@@ -150,6 +165,7 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int
   __shared__ int32_t red_live[kThreads / 64];
   __shared__ int32_t red_tiles;
   __shared__ int32_t q_lo[4], q_hi[4];
+  __shared__ pa_term terms_s[PA_MAX_TERMS];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -167,6 +183,9 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int
     q_orig[tid] = pred.perm_q ? pred.perm_q[r] : r;
   }
   if (tid == 0) red_tiles = 0;
+#pragma unroll
+  for (int i = 0; i < PA_MAX_TERMS; ++i)  // (constant indices into the argument block)
+    if (tid == i) terms_s[i] = pred.terms[i];
   __syncthreads();
   if (wave < n_rg) {
     // the row groups' ranges (their rows, one per lane; lanes past them repeat)
@@ -199,7 +218,8 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int
       // a chunk of columns in order that is live or dead as a whole (uniform: no barrier)
       rw.k0 = c0;
       rw.k1 = min(c0 + kChunk, N) - 1;
-      const Verdict v = pred_verdict(pred, rw, [](int32_t p) -> int { return p == 1 ? 1 : -1; });
+      const Verdict v =
+          pred_verdict(terms_s, pred.n_include, pred.n_exclude, rw, [](int32_t p) -> int { return p == 1 ? 1 : -1; });
       if (v != kMixed) {
         const int cols = rw.k1 - c0 + 1, tiles = cols >> log2a;
         if (tid < tiles) codes[(int64_t)qb * nk + (c0 >> log2a) + tid] = v == kLive ? all_code : 0u;
@@ -228,16 +248,19 @@ __global__ __launch_bounds__(kThreads) void classify_kernel(const Pred pred, int
         r.k0 = c0 + wave * 64;
         r.k1 = min(c0 + wave * 64 + 64, N) - 1;
       }
+      // columns from all over the sequence (a random permutation): hardly a block is decided
+      const bool wide = pred.perm_kv && r.k1 - r.k0 >= N >> 1;
       for (int g = 0; g < n_rg; ++g) {
         const int32_t qo = q_orig[g * rg_rows + (lane & (rg_rows - 1))];
         r.q0 = q_lo[g];
         r.q1 = q_hi[g];
-        const Verdict v = pred_verdict(pred, r, [&](int32_t p) -> int {
+        auto same = [&](int32_t p) -> int {
           const int32_t rq = qo % p, rk = ko % p;
           const int32_t rq0 = __builtin_amdgcn_readfirstlane(rq), rk0 = __builtin_amdgcn_readfirstlane(rk);
           if (__ballot(rq != rq0 || rk != rk0) != 0ull) return -1;
           return rq0 == rk0 ? 1 : 0;
-        });
+        };
+        const Verdict v = wide ? kMixed : pred_verdict(terms_s, pred.n_include, pred.n_exclude, r, same);
         bool any = v == kLive, all = v == kLive;
         if (v == kMixed) {
           all = true;
