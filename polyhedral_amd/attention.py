@@ -95,6 +95,14 @@ class Launch:
         self.entry = entry
         self._ref = ctypes.byref(args)
 
+    @property
+    def device_kernel(self):
+        """The HIP kernel that the launch runs."""
+        if self.entry == "pa_attn_fwd_tile":
+            return "attn_tile_kernel" if self.args.BQ >= 64 else "attn_narrow_kernel"
+        return {"run": "attn_run_kernel", "stream": "attn_stream_kernel",
+                "wsplit": "attn_wsplit_kernel"}.get(self.kernel, "attn_fwd_kernel")
+
     def __call__(self):
         _lib.check(getattr(_lib.lib(), self.entry)(self._ref, _lib.stream_of(self.out)), self.entry)
         return self.out

@@ -137,3 +137,30 @@ def test_narrow_blocks_of_a_short_sequence(gpu, N):
         lists, wave, bits = _built(numpy_mask("causal"), N, 16, 16, gpu)
         for kb in (bits, None):
             _both(q, k, v, lists, triton_params("causal"), 16, 16, kv_wave_bits=wave, kv_bits=kb)
+
+
+@pytest.mark.parametrize("dtype,D,BQ,A,ext,want", [
+    (torch.float16, 64, 128, 32, {}, "attn_tile_kernel"),
+    (torch.bfloat16, 128, 64, 64, {}, "attn_tile_kernel"),
+    (torch.bfloat16, 128, 128, 128, {}, "attn_tile_kernel"),
+    (torch.float16, 128, 32, 16, {}, "attn_narrow_kernel"),
+    (torch.bfloat16, 64, 16, 16, {}, "attn_narrow_kernel"),
+    (torch.bfloat16, 128, 128, 32, {}, "attn_stream_kernel"),
+    (torch.bfloat16, 128, 128, 32, dict(kernel="general"), "attn_fwd_kernel"),
+    (torch.float16, 64, 64, 64, dict(kernel="general"), "attn_fwd_kernel"),
+    (torch.float32, 64, 64, 64, {}, "attn_wsplit_kernel"),
+    (torch.float32, 64, 16, 16, {}, "attn_fwd_kernel"),
+    (torch.float16, 64, 64, 64, dict(perm=True), "attn_tile_kernel"),                   # the mask alone relabelled
+    (torch.float16, 64, 64, 64, dict(perm=True, gather_kv=True), "attn_fwd_kernel"),    # through a table
+    (torch.float16, 64, 64, 64, dict(perm=True, gather_kv=True, residue=8), "attn_tile_kernel"),
+    (torch.float16, 64, 16, 16, dict(gather_mult=2), "attn_fwd_kernel"),
+])
+def test_the_kernel_a_call_takes(gpu, dtype, D, BQ, A, ext, want):
+    N = 512
+    q = torch.zeros(1, N, D, dtype=dtype, device=gpu)
+    bi = pindex.build(numpy_mask("window-128"), N, BQ, A)
+    ext = dict(ext)
+    if ext.pop("perm", False):
+        ext["perm_q"] = torch.from_numpy(op.residue_perm(N, 8)).to(gpu)
+    launch = pattn.prepare(q, q, q, *pindex.to_cuda(bi), *triton_params("window-128"), BQ, A, **ext)
+    assert launch.device_kernel == want
