@@ -267,10 +267,11 @@ typedef struct pa_attn_args {
 int pa_attn_fwd(const pa_attn_args* args, void* stream);
 
 /* pa_attn_fwd_tile: the same attention by the kernels for f16 / bf16 block lists as they are
- * (no step descriptors; kv_wave_bits and the bitmaps optional), any tile, with any gather_q / scatter_o / prev_o / order, and gather_kv through the
- * closed-form residue basis only; gather_mult <= 1, no kv_steps, run_groups or wave_split,
- * and N * row stride of k and v below 4 GiB.
- * Results within the rounding of P to 16 bits of pa_attn_fwd's without kv_steps. */
+ * (no step descriptors; kv_wave_bits and the bitmaps optional), any tile, with any gather_q /
+ * scatter_o / prev_o / order, and gather_kv through the closed-form residue basis only;
+ * gather_mult <= 1, no kv_steps, run_groups or wave_split, and N * row stride of k and v
+ * below 4 GiB.  Results within the rounding of P to 16 bits of pa_attn_fwd's without kv_steps,
+ * NaN and infinities in the same places. */
 int pa_attn_fwd_tile(const pa_attn_args* args, void* stream);
 
 /* A two-piece disjoint split in ONE persistent launch (no counterpart in the reference,

@@ -18,9 +18,13 @@
 //    16 different units of the 256-byte window;
 //  * the list is held 32 steps at a time, a segment per lane.
 //
-// What bounds it: every wave reads its own K and V rows (8 KB per 16 x 32 pairs at D = 128,
-// from the L1 and L2) and its scalar and softmax work per step covers only 8 or 16 short
-// MFMAs; four waves per SIMD (118 registers) at D = 64 and two (186) at D = 128.  Against
+// What bounds it: the latency of a wave's step, whose loads are issued one step ahead and all
+// waited for.  Lattice-8 in its basis, 8 heads x 8192, 16x16 tiles, D = 64, is one round of
+// work-groups; a step of its longest lists takes some 2900 clocks, of which the 8 MFMAs are
+// 128, and waves wait on a counter 56% of theirs (2.5 waves per SIMD on average, VALU 23%,
+// matrix cores 7% of the SIMDs' clocks).  Every wave reads its own K and V rows: 8 KB per 16 x
+// 32 pairs at D = 64 and 16 KB at D = 128, from the L1 and L2.  118 registers at D = 64 (four
+// waves per SIMD), 182 at D = 128 (two).  Against
 // attn_fwd_kernel, f16: lattice-8 in its basis, 8 heads x 8192, 16x16 tiles, D = 64 211 ->
 // 45 us (191 live TFLOP/s); window 256, 8 x 8192: 16x16 140 -> 29 us, D = 128 286 -> 54;
 // 32x32 89 -> 31, D = 128 171 -> 58; causal, 8 x 2048: 16x16 128 -> 42, D = 128 241 -> 79;
@@ -279,7 +283,8 @@ void attn_narrow_kernel(const AttnK a, int units, int groups) {
   Data d0{}, d1{};
   // The step's V rows are in LDS and its K rows in registers once everything issued is done.
   // The memory clobber keeps the ring's reads on their side of the wait (no barrier does),
-  // and the last step's are done before the next DMA into their stage; the uses make the compiler's own wait fall here, before the next step's loads.
+  // and the last step's are done before the next DMA into their stage; the uses make the
+  // compiler's own wait fall here, before the next step's loads.
   auto arrive = [&](const Data& d) __attribute__((always_inline)) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 #pragma unroll

@@ -5,29 +5,34 @@
 // _attn_fwd, gpu/triton_attn.py:62-182): scores transposed (S^T = K Q^T) on 32x32x16 MFMAs,
 // online softmax with the finite -1e30 sentinel and a lazy rescale, probabilities rounded
 // to 16 bits only as MFMA operands (their sum is taken in fp32 before), the l > 0 guard, and
-// the log-sum-exp merge with a previous partial (narrower query blocks: attn_narrow.hip).  attn_fwd_kernel stages K and V through
-// registers and keeps the rest: f32, K / V gathered through a permutation table,
-// class-B emulation.
+// the log-sum-exp merge with a previous partial (narrower query blocks: attn_narrow.hip).
+// attn_fwd_kernel stages K and V through registers and keeps the rest: f32, K / V gathered
+// through a permutation table, class-B emulation.
 //
 // A work-group is RG row groups (one wave of 32 query rows each; all of the query block's, or
 // with H = 2 half of them) times KG key groups.  Key group g takes the 64-column steps g,
-// g + KG, ... of the query block's list, its K and V rows by LDS DMA into a two-stage ring of its own (layout in lds_rows.hpp), the
-// next step's while this one is computed, behind one wait and one barrier per step.  The key
-// groups' states (max, sum, O^T) are merged through LDS at the end.
+// g + KG, ... of the query block's list, its K and V rows by LDS DMA into a two-stage ring of
+// its own (layout in lds_rows.hpp), the next step's while this one is computed, behind one
+// wait and one barrier per step.  The key groups' states (max, sum, O^T) are merged through
+// LDS at the end.
 //
 // What bounds it: at D = 64 a step's 16 MFMAs take 512 clocks of a SIMD and its exponentials,
-// maxima, sums and packing about 850, so the VALU, as far as three waves per SIMD overlap
-// (causal, 32 heads x 8192, f16: 375 us, 730 TFLOP/s, about 1500 clocks per wave's step); on
-// short lists an item's start and end.  Against attn_fwd_kernel: that case 798 us; 8 heads x
+// maxima, sums and packing about 850.  With every CU full (causal, 32 heads x 8192, f16: 375
+// us, 730 TFLOP/s, about 1500 clocks per wave's step) the VALU is busy 61% of the SIMDs'
+// clocks and the matrix cores 33%, less than half of that at the same time: the issue of the
+// two, hardly overlapped (2.2 waves per SIMD on average).  On smaller launches the latency of
+// a wave's step: causal, 8 x 4096, has 1.1 waves per SIMD, VALU 26%, matrix cores 13%, and
+// waits for its longest lists; lattice-8 in its basis, 8 x 16384, 1.5 waves, 40% and 20%.
+// Against attn_fwd_kernel: the first case 798 us; 8 heads x
 // 4096 causal, 128x128 tiles, f16, D = 64 (no bitmaps) 138 -> 44 us; lattice-8 in its basis,
 // 8 heads x 16384, 128x32 tiles 155 -> 64 us; causal, bf16, D = 128, 8 x 4096, 128x128 tiles
 // 209 -> 77 us.  A step's scalar work decides much of it (the scalar unit is shared by the
 // SIMDs): the list read entry by entry, with its codes worked out per step, took 64 us where
 // 16 steps at a time took 55.
 //
-// The list is held 16 steps at a time, a 16-column segment per lane; a partial block's mask word (32 columns of the lane's query row)
-// is loaded from the bitmaps one step ahead, or evaluated from the predicate when the index
-// has no bitmaps.
+// The list is held 16 steps at a time, a 16-column segment per lane; a partial block's mask
+// word (32 columns of the lane's query row) is loaded from the bitmaps one step ahead, or
+// evaluated from the predicate when the index has no bitmaps.
 #include <type_traits>
 
 #include "lds_rows.hpp"
@@ -38,7 +43,8 @@ namespace {
 template <int D, int KG>
 constexpr int tile_smem_bytes() { return KG * 4 * 64 * Rows<D>::ROW; }
 
-// Waves per SIMD that the registers allow (168 and 248 in use, no spills).
+// Waves per SIMD that the registers allow (163 to 168 and 246 to 254 in use by the
+// instantiations, none spilled; 2 to 27 scalars are).
 template <int D>
 constexpr int tile_waves() { return D == 64 ? 3 : 2; }
 
@@ -71,7 +77,8 @@ void attn_tile_kernel(const AttnK a) {
   // sequence, and the longest should not be the last to start: 456 -> 375 us for 32 heads of
   // 8192 in f16, D = 64.  Up to 1024 work-groups, which mostly start at once, are also dealt
   // to the CUs long with short: 69.5 -> 64.5 us for the lattice-8 mask below; beyond that it
-  // costs 3% of L2 reuse.)
+  // costs 3% of L2 reuse.  An order that the caller gives, as a split plan's, is taken as it
+  // is.)
   const int p = a.qblock_order ? p_lin : np - 1 - (gridDim.x <= 1024 ? snake(p_lin, np) : p_lin);
   const int qb = a.qblock_order ? ((cint*)a.qblock_order)[p / H] : p / H;
   const int wb = (p % H) * RG + w;  // this wave's row group in the query block
@@ -486,7 +493,8 @@ int launch_tile_t(const AttnK& a, hipStream_t s) {
     if (e != hipSuccess) return hip_fail(e, "hipFuncSetAttribute(attn_tile_kernel)");
     if (dev < 64) configured |= 1ull << dev;
   }
-  hipLaunchKernelGGL((attn_tile_kernel<T, D, RG, KG, H>), dim3((unsigned)(H * a.total_wg)), dim3(64 * RG * KG), smem, s, a);
+  hipLaunchKernelGGL((attn_tile_kernel<T, D, RG, KG, H>), dim3((unsigned)(H * a.total_wg)), dim3(64 * RG * KG), smem,
+                     s, a);
   PA_LAUNCH_CHECK("attn_tile_kernel");
   return PA_OK;
 }

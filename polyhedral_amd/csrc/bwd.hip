@@ -245,9 +245,13 @@ __device__ __forceinline__ void store_rows(const BwdK& a, char* smem, const f32x
 //
 // What bounds it: on long lists the MFMAs (causal, 32 heads x 8192, D = 128, bf16: both
 // kernels together 1.9 ms, 1.0 PFLOP/s of the 14 D per pair they issue, 80% of a large
-// torch matmul's rate); on short lists each item's start and end and its rows' bytes.  Two
-// waves per SIMD is what the registers allow at D = 128 (dK and dV take 128 of 256; K in
-// registers, V in LDS but for one fragment, address halves recomputed: 251 without spills).
+// torch matmul's rate); on short lists each item's start and end and its rows' bytes (band and
+// lattice below, lists of about 7 tiles: matrix cores busy 24% of the SIMDs' clocks in the
+// band's launches and 33% in the lattice's).  Two waves per SIMD is what the registers allow
+// at D = 128 (dK and dV take 128 of 256; K in registers, V in LDS but for one fragment, address
+// halves recomputed: 247 with bitmaps, 251 without, none spilled).  Without bitmaps at D = 64
+// three waves with 8 spilled registers take 360 us where two with none take 370 (causal, 15 x
+// 8192).
 // Splitting a tile by quadrants replaced a pair of waves per 32 keys, one for P and dV and
 // one for dP and dK, that met at a barrier in the middle of every tile with P in LDS
 // (D = 128), and register-staged tiles that evaluated the mask and waited for each tile

@@ -486,16 +486,22 @@ __device__ __forceinline__ float group_sum(float x) {
 // at different times.  The dot product is reduced over the group by DPP; the probability is
 // then in the lanes that hold the row's V, which keep their own running maximum, sum and output
 // and meet only at the end.  The live keys are listed as in decode_kernel, in a ring of 128
-// entries per wave; the ring starts a 64-key block at another place in neighbouring waves,
-// or all of them read the same part of a 16-KiB block at a time, which is the same channels'
-// in every head (110 -> 105 us in the first case below, 97 -> 88 with the next), with
-// non-temporal loads (a cached row is used once), and K's loads ahead of V's (88 -> 86).
+// entries per wave; with 256-byte rows, whose batch is half of a 64-key block, the ring
+// starts a block with the other half in neighbouring waves, or all of them read the same part
+// of a 16-KiB block at a time, which is the same channels' in every head (110 -> 105 us in the
+// first case below, 97 -> 88 with the next; a batch of 128-byte rows is a whole block and
+// starts at its first key: batches of 4 rows, which rotate there too, take 46.3 us against
+// 46.7 of 256 heads x 3977 keys and are up to 10% slower on windows in a basis), non-temporal
+// loads (a cached row is used once), and K's loads ahead of V's (88 -> 86).
 // Against decode_kernel, whose lanes read a K row each, wait for V in LDS and load nothing
 // meanwhile (us, both kernels of a call; bf16, D = 128): 256 heads x 3977 keys, causal 97.5 ->
 // 85.1 (5.4 -> 6.1 TB/s), 200 x 4100 106.7 -> 76.2, 32 x 65000 193 -> 162, 32 x 16011 51.2 ->
 // 49.1, band-256 | lattice-16 in its basis at 32 x 16011 21.2 -> 16.4, window 300 at 64 x 3977
 // 16.8 -> 14.1, D = 64 at 256 x 3977 51.4 -> 48.2; batches of 4 rows are as fast at the
-// largest and up to 1 us slower at the smallest, of 16 rows slower throughout.
+// largest and up to 1 us slower at the smallest, of 16 rows slower throughout.  Slower than
+// decode_kernel was only on the smallest calls in a residue basis, which it took without a
+// list: 64 to 4000 keys at 1 to 32 heads 9.3 -> 9.5 us, at D = 64 9.4 -> 10.1 (prepared once;
+// by themselves such calls take the host 19 us).
 template <typename T, int D>
 __global__ __launch_bounds__(64 * kOneWaves) __attribute__((amdgpu_waves_per_eu(4)))
 void decode_one_kernel(const DecK a) {
@@ -539,7 +545,8 @@ void decode_one_kernel(const DecK a) {
 
   int head = 0, nlist = 0;  // the ring's first entry and length (at most B - 1 + 64)
   uint32_t g = (uint32_t)split + (uint32_t)(w >> 2) * (uint32_t)a.n_split;
-  // the key of its 64 that lane 0 stands for, another batch's in neighbouring waves
+  // the key of its 64 that lane 0 stands for, another batch's in neighbouring waves (0 where
+  // a batch is a whole block)
   const int rot = ((w + split + (int)bh) * B) & 63;
   struct Batch {
     du4 k[NI], v[NI];
